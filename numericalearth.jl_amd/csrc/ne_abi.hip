@@ -703,7 +703,7 @@ static int model_update_state(ne_model* m, double dt_frazil, hipStream_t s, hipE
     NetOut n = net_out(d.net);
     RadOut ro = rad_out(d.radiative);
     View3<double> frazil = view<double>(d.frazil_heat);
-    const uint8_t* flags = after_step ? m->freeze_flags : nullptr;
+    uint8_t* flags = after_step ? m->freeze_flags : nullptr;
     hipError_t e;
     if (d.precision == NE_FP64) {
         AtmosDev<double> a = atmos_dev<double>(d.atmosphere);
@@ -872,9 +872,9 @@ int ne_model_create(ne_ctx* c, const ne_model_desc* desc, ne_model** out, void* 
         ne_model_destroy(m);
         return NE_ERR_DEVICE;
     }
-    // every column is visited until a step's last stage has flagged them; the residual starts
-    // at zero (creation is never inside a captured graph, so the fills may be memsets)
-    if (hipMemsetAsync(m->freeze_flags, 1, freeze_flag_bytes(*desc), as_stream(stream)) != hipSuccess ||
+    // no column is flagged between steps (update_state outside a step visits every one); the residual
+    // starts at zero (creation is never inside a captured graph, so the fills may be memsets)
+    if (hipMemsetAsync(m->freeze_flags, 0, freeze_flag_bytes(*desc), as_stream(stream)) != hipSuccess ||
         hipMemsetAsync(m->residual, 0, residual_bytes(*desc), as_stream(stream)) != hipSuccess ||
         hipMemsetAsync(m->deferred, 0, sizeof(int), as_stream(stream)) != hipSuccess ||
         launch_beer_factors(grid_dev(desc->grid), desc->params.first_absorption_coefficient,

@@ -140,7 +140,8 @@ hipError_t enqueue(ne_batch* b, double dt, hipStream_t s, ne_counters* counters)
 }
 
 template <typename Real>
-BatchRec<Real> member_record(const ne_model* m, const double* atimes_dev, const double* rtimes_dev) {
+BatchRec<Real> member_record(const ne_model* m, const double* atimes_dev, const double* rtimes_dev,
+                             int64_t tile_levels) {
     const ne_model_desc& d = m->d;
     BatchRec<Real> r;
     memset(&r, 0, sizeof(r));
@@ -174,6 +175,7 @@ BatchRec<Real> member_record(const ne_model* m, const double* atimes_dev, const 
     r.freeze_flags = m->freeze_flags;
     r.residual = m->residual;
     r.beer = m->beer;
+    r.levels = stage_levels(r.g, tile_levels);
     r.atimes = atimes_dev;
     r.rtimes = rtimes_dev;
     r.nat = (int)m->atimes.size();
@@ -195,15 +197,22 @@ int rebuild(ne_batch* b, hipStream_t s) {
     const int n = (int)b->members.size();
     // work lists and snapshot times on the host
     std::vector<WorkItem> stage[2][3], surface[3], solve[3][3];
+    std::vector<int> below_top[2][3];   // chunks above each stage item's in its tile
     std::vector<double> times;
     std::vector<size_t> aoff(n), roff(n);
+    int64_t tile_levels = 0;   // of the whole batch: its members share the chip
+    for (const ne_model* m : b->members) tile_levels += stage_tile_levels(grid_dev(m->d.grid));
     for (int k = 0; k < n; k++) {
         const ne_model* m = b->members[k];
         const ne_grid& g = m->d.grid;
         const int tc = m->d.params.radiative_forcing == NE_RADIATIVE_FORCING_TWO_COLOR ? 1 : 0;
+        const int chunks = level_chunks(g.Nz, stage_levels(grid_dev(g), tile_levels));
         for (int c = 0; c < 3; c++) {
-            int nt = batch_tiles_x(g.Nx) * batch_tiles_y(g.Ny, TILE_ROWS[c]);
-            for (int t = 0; t < nt; t++) stage[tc][c].push_back(WorkItem{k, t});
+            int nt = batch_tiles_x(g.Nx) * batch_tiles_y(g.Ny, TILE_ROWS[c]) * chunks;
+            for (int t = 0; t < nt; t++) {
+                stage[tc][c].push_back(WorkItem{k, t});
+                below_top[tc][c].push_back(chunks - 1 - t % chunks);
+            }
         }
         int path = flux_path(m->d.params);
         int cols = g.Nx * g.Ny;
@@ -217,6 +226,21 @@ int rebuild(ne_batch* b, hipStream_t s) {
         roff[k] = times.size();
         times.insert(times.end(), m->rtimes.begin(), m->rtimes.end());
     }
+    // each XCD's part of a stage list: its uppermost chunks of levels first, as in the single-model kernel
+    for (int tc = 0; tc < 2; tc++)
+        for (int c = 0; c < 3; c++) {
+            std::vector<WorkItem>& w = stage[tc][c];
+            const size_t part = (w.size() + NXCD - 1) / NXCD;
+            std::vector<size_t> order(w.size());
+            for (size_t q = 0; q < w.size(); q++) order[q] = q;
+            for (size_t q = 0; q < w.size(); q += part)
+                std::stable_sort(order.begin() + q, order.begin() + std::min(q + part, w.size()), [&](size_t x, size_t y) {
+                    return below_top[tc][c][x] < below_top[tc][c][y];
+                });
+            std::vector<WorkItem> sorted(w.size());
+            for (size_t q = 0; q < w.size(); q++) sorted[q] = w[order[q]];
+            w.swap(sorted);
+        }
     Layout L;
     size_t off = 0;
     L.recs = off;
@@ -268,7 +292,7 @@ int rebuild(ne_batch* b, hipStream_t s) {
     for (int k = 0; k < n; k++) {
         const ne_model* m = b->members[k];
         recs[k] = member_record<Real>(m, m->atimes.empty() ? nullptr : tdev + aoff[k],
-                                      m->rtimes.empty() ? nullptr : tdev + roff[k]);
+                                      m->rtimes.empty() ? nullptr : tdev + roff[k], tile_levels);
     }
     if (!times.empty()) memcpy(H + L.times, times.data(), times.size() * sizeof(double));
     auto put = [&](size_t o, const std::vector<WorkItem>& w, WorkItem** view, int* count) {

@@ -23,8 +23,8 @@ struct ne_model {
     void* T2 = nullptr;
     void* S2 = nullptr;
     ne_view vT1, vS1, vT2, vS2;
-    // one byte per column, written by the step's last RK stage: 1 where a cell of the column is
-    // below its freezing point (or not known), so the freeze clamp that follows visits only those
+    // one byte per column, set by the step's last RK stage where a cell of the column is below its
+    // freezing point, so the freeze clamp that follows visits only those and clears them
     uint8_t* freeze_flags = nullptr;
     // rounding residual of the FP32 state (residual_bytes): per tile, the running compensated
     // totals Σ V·(x − stored) of T and S (sum, compensation, sum, compensation)
@@ -150,7 +150,7 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
                                  const double* fj, const RadDev<Real>& r, const double* rfi, const double* rfj,
                                  View3<Real> T, View3<const Real> S, View3<const Real> u, View3<const Real> v,
                                  const FluxOut& out, const NetOut& n, const RadOut& ro, View3<double> frazil,
-                                 double dt_frazil, const uint8_t* freeze_flags, ne_counters* c, int* deferred,
+                                 double dt_frazil, uint8_t* freeze_flags, ne_counters* c, int* deferred,
                                  hipStream_t s);
 // deferred (FP32 storage; nullptr: none): count + one int per column for the columns K1 leaves to
 // its second kernel; the τ kernel, which runs after both, clears the count.
@@ -208,7 +208,7 @@ double* budget_noalloc_scratch(int device);
 int64_t budget_blocks(const GridDev& g);
 hipError_t launch_budget_noalloc(double* partial, const GridDev& g, View3<const double> c, double weight,
                                  double* out, hipStream_t s);
-// Rounding residual of an FP32 state: one slot per tile (T sum, T compensation, S sum,
+// Rounding residual of an FP32 state: one slot per tile and chunk of levels (T sum, T compensation, S sum,
 // S compensation), into which the block of the step's last stage adds the tile's Σ V·(x −
 // stored); the number of slots a model keeps, and their fixed-order sum into out[4].
 constexpr int RESIDUAL_SLOT = 4;
@@ -223,6 +223,11 @@ hipError_t launch_halo_fill(const GridDev& g, View3<Real> c, int Hx, int Hy, int
 hipError_t launch_stream_probe(const double* const* in, int n_in, double* const* out, int n_out, int64_t n,
                                hipStream_t s);
 int64_t residual_slots(const GridDev& g);
+// Levels of a tile that one block of the stage and tendency kernels takes, and the number of such
+// chunks in a column of Nz levels.
+int64_t stage_tile_levels(const GridDev& g);
+int stage_levels(const GridDev& g, int64_t tile_levels);
+__host__ __device__ inline int level_chunks(int Nz, int levels) { return (Nz + levels - 1) / levels; }
 hipError_t launch_residual_reduce(const double* residual, const GridDev& g, double* out, hipStream_t s);
 
 // ---------------------------------------------------------------------------
@@ -253,6 +258,7 @@ struct BatchRec {
     uint8_t* freeze_flags;  // the member's freeze flags (written by stage 3, read by K2)
     double* residual;       // the member's rounding residual (running totals per tile)
     const double* beer;     // the member's Beer's-law factors (two-colour forcing)
+    int levels;             // levels per block of the stages (stage_levels)
     const double* atimes;   // device copies of the snapshot times
     const double* rtimes;
     int nat, nrt;

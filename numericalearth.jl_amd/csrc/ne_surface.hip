@@ -582,11 +582,16 @@ __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const 
                                                         const View3<const Real>& S, const FluxOut& f,
                                                         const NetOut& n, const RadOut& ro,
                                                         const View3<double>& frazil, double dt_frazil,
-                                                        const uint8_t* __restrict__ freeze_flags, double Qt,
+                                                        uint8_t* __restrict__ freeze_flags, double Qt,
                                                         double Qv, double Jv, double Ts_C, int i, int j) {
     // after a step, only columns its last stage flagged can hold a cell below freezing; the
     // others would run the clamp without a change and with dQ = 0 (the same +0.0)
-    const bool visit = freeze_flags == nullptr || freeze_flags[(int64_t)i + (int64_t)j * g.Nx] != 0;
+    bool visit = freeze_flags == nullptr;
+    if (!visit) {
+        uint8_t& flag = freeze_flags[(int64_t)i + (int64_t)j * g.Nx];
+        visit = flag != 0;
+        if (visit) flag = 0;   // the stages only set flags
+    }
     double dQ = visit ? freeze_column<Real>(g, p, T, S, i, j, dt_frazil) : 0.0;
     if (frazil.p) frazil.at2(i, j) = dQ;
 
@@ -640,7 +645,7 @@ surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __
                       const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
                       const double* __restrict__ rfj, View3<Real> T, View3<const Real> S, View3<const Real> u,
                       View3<const Real> v, FluxOut out, NetOut n, RadOut ro, View3<double> frazil, double dt_frazil,
-                      const uint8_t* __restrict__ freeze_flags, ne_counters* counters, int* deferred) {
+                      uint8_t* __restrict__ freeze_flags, ne_counters* counters, int* deferred) {
     int i = blockIdx.x * BX + threadIdx.x;
     int j = blockIdx.y * KBY + threadIdx.y;
     if (out.iters.p && !Defer) {
@@ -685,7 +690,7 @@ surface_deferred_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* 
                         const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
                         const double* __restrict__ rfj, View3<Real> T, View3<const Real> S, View3<const Real> u,
                         View3<const Real> v, FluxOut out, NetOut n, RadOut ro, View3<double> frazil,
-                        double dt_frazil, const uint8_t* __restrict__ freeze_flags, ne_counters* counters,
+                        double dt_frazil, uint8_t* __restrict__ freeze_flags, ne_counters* counters,
                         const int* __restrict__ deferred) {
     const int count = deferred[0];   // the same for every work-item: nothing writes it meanwhile
     // rounds of one column per work-item, uniform over the block (the counters synchronise it)
@@ -981,7 +986,7 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
                                  const double* fj, const RadDev<Real>& r, const double* rfi, const double* rfj,
                                  View3<Real> T, View3<const Real> S, View3<const Real> u, View3<const Real> v,
                                  const FluxOut& out, const NetOut& n, const RadOut& ro, View3<double> frazil,
-                                 double dt_frazil, const uint8_t* freeze_flags, ne_counters* c, int* deferred,
+                                 double dt_frazil, uint8_t* freeze_flags, ne_counters* c, int* deferred,
                                  hipStream_t s) {
     const int path = flux_path(p);
     const dim3 grid = grid2d(g.Nx, g.Ny);
@@ -1010,13 +1015,13 @@ template hipError_t launch_surface_update<double>(const GridDev&, const ne_param
                                                   const double*, View3<double>, View3<const double>,
                                                   View3<const double>, View3<const double>, const FluxOut&,
                                                   const NetOut&, const RadOut&, View3<double>, double,
-                                                  const uint8_t*, ne_counters*, int*, hipStream_t);
+                                                  uint8_t*, ne_counters*, int*, hipStream_t);
 template hipError_t launch_surface_update<float>(const GridDev&, const ne_params&, const AtmosDev<float>&,
                                                  const double*, const double*, const RadDev<float>&, const double*,
                                                  const double*, View3<float>, View3<const float>,
                                                  View3<const float>, View3<const float>, const FluxOut&,
                                                  const NetOut&, const RadOut&, View3<double>, double,
-                                                 const uint8_t*, ne_counters*, int*, hipStream_t);
+                                                 uint8_t*, ne_counters*, int*, hipStream_t);
 
 hipError_t launch_surface_tau(const GridDev& g, const ne_params& p, const FluxOut& f, const NetOut& n,
                               int* deferred, hipStream_t s) {

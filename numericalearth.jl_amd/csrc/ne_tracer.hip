@@ -2,11 +2,14 @@
 // with the top flux boundary condition and the split Runge-Kutta stage update.
 //
 // Tiling (gfx950): a block of 64·TR work-items = TR wavefronts (TR = 4 for one model) owns
-// a tile of 63 × TR columns and marches up the active levels. At each level the tile's T
-// and S plane plus a 3-cell halo (69 × (TR+6) cells) is staged in LDS; every x- and y-face
-// flux of the tile is reconstructed once (lane ℓ of wavefront r owns the west face of
-// column ℓ and the south face of row r, lane 63 only a face; T, then S), written to LDS,
-// and differenced by the owning cell. The vertical face flux at the top of level k is
+// a tile of 63 × TR columns and marches up its active levels (all of them, or a chunk of them where
+// the grid has too few tiles to fill the chip: stage_levels). At each level the tile's T and S plane
+// plus a 3-cell halo (69 × (TR+6) cells) is staged in LDS, the tile's own cells from the columns'
+// register windows and the halo from memory (loading the own cells a second time, a third of the
+// plane, and keeping the set-up's conditional loads took the FP64 stage of 1440×560×10 to 146 µs
+// against 136); every x- and y-face flux of the tile is reconstructed once (lane ℓ of wavefront r
+// owns the west face of column ℓ and the south face of row r, lane 63 only a face; T, then S),
+// written to LDS, and differenced by the owning cell. The vertical face flux at the top of level k is
 // carried in registers as the bottom flux of level k+1, with the column's vertical stencil
 // in a register window. Row-dependent values are wavefront-uniform (one wavefront per row)
 // and kept in scalar registers. Tiles are ordered so that each XCD (blocks are dealt
@@ -81,15 +84,16 @@ struct TileShared {
     R fxT[TR * TW], fxS[TR * TW];
     R fyT[(TR + 1) * TC], fyS[(TR + 1) * TC];
     int km[PN];
-    int kstart;
     double resid[2 * TR];   // the rows' rounding residuals of T and S (FP32 state's last stage)
 };
 
 __host__ __device__ inline int tiles_x(int Nx) { return (Nx + TC - 1) / TC; }
 __host__ __device__ inline int tiles_y(int Ny, int tr) { return (Ny + tr - 1) / tr; }
-inline int grid_blocks(int Nx, int Ny) {
-    int n = tiles_x(Nx) * tiles_y(Ny, PLAIN_TR);
-    return ((n + NXCD - 1) / NXCD) * NXCD;
+
+// Blocks of the single-model kernel: every tile's levels in chunks of `levels`.
+inline int grid_blocks(const GridDev& g, int levels) {
+    int n = tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR);
+    return ((n + NXCD - 1) / NXCD) * NXCD * level_chunks(g.Nz, levels);
 }
 
 // Face order at level k from the three thresholds of its stencil: the face is
@@ -100,6 +104,12 @@ inline int grid_blocks(int Nx, int Ny) {
 constexpr uint32_t NEVER_LEVEL = 1023u;
 __device__ __forceinline__ int order_at(int k, uint32_t P) {
     return (k >= (int)(P & 1023u) ? 1 : 0) + (k >= (int)((P >> 10) & 1023u) ? 1 : 0) + (k >= (int)(P >> 20) ? 1 : 0);
+}
+
+// Face order at the top of level k of a column with active levels kmin … Nz-1.
+__device__ __forceinline__ int z_order(int k, int kmin, int Nz) {
+    return (k >= kmin && k <= Nz - 2 ? 1 : 0) + (k >= kmin + 1 && k <= Nz - 3 ? 1 : 0) +
+           (k >= kmin + 2 && k <= Nz - 4 ? 1 : 0);
 }
 
 __device__ __forceinline__ uint32_t thresholds(const int* km, int stride) {
@@ -182,7 +192,9 @@ __device__ __forceinline__ DD dd_add(DD a, DD b) {
     return r;
 }
 
-// One tile (columns i0 … i0+62, rows j0 … j0+TR-1) marched over its active levels.
+// One tile (columns i0 … i0+62, rows j0 … j0+TR-1) marched over its active levels among k0 … k1-1.
+// A chunk that starts above the tile's lowest active level reconstructs the flux through its
+// bottom face itself, from the same cells as the chunk below does: the same bits.
 // MODE 0: c_out = c0 + beta_dt·G(c_in) on active cells. MODE 1: write G (0 on inactive
 // cells). Every work-item of the block calls this with the same tile. Every address is a
 // 32-bit byte offset from a uniform base (the host checks that each view spans < 4 GiB),
@@ -195,14 +207,17 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
                                           const Real* __restrict__ Tin, const Real* __restrict__ Sin, Real* Tout,
                                           Real* Sout, const double* __restrict__ JT, const double* __restrict__ JS,
                                           const double* __restrict__ Jw, const TracerForcing& F, double beta_dt,
-                                          int i0, int j0, bool stochastic = false, uint32_t seed = 0u) {
+                                          int i0, int j0, int k0, int k1, bool stochastic = false,
+                                          uint32_t seed = 0u) {
     typedef Real R;
     constexpr int PXW = TileShared<R, TR>::PXW;
     constexpr int PN = TileShared<R, TR>::PN;
     constexpr int NTHR = TW * TR;
-    constexpr int NPL = (PN + NTHR - 1) / NTHR;   // plane cells staged per work-item
+    // halo cells of the plane: three full rows below and above the tile, three cells on each side
+    // of its rows (the tile's own cells come from the work-items' vertical windows)
+    constexpr int NH = 6 * PXW + 6 * TR;
+    constexpr int NPL = (NH + NTHR - 1) / NTHR;   // halo cells staged per work-item
     constexpr uint32_t ES = sizeof(R);
-    constexpr int NEVER = 1 << 30;
     const int lane = threadIdx.x;
     const int row = wave_uniform((int)threadIdx.y);   // one wavefront per row
     const int tid = lane + row * TW;
@@ -215,28 +230,36 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
         int64_t c = g.column(i0 - 3 + pi, j0 - 3 + pj);
         sh.km[n] = c >= 0 ? g.kmin[c] : KMIN_OUTSIDE;
     }
-    if (tid == 0) sh.kstart = Nz;
     __syncthreads();
     const int ci = i0 + lane, cj = j0 + row;
     const bool cell = lane < TC && ci < g.Nx && cj < g.Ny;
-    const int mykmin = cell ? sh.km[(row + 3) * PXW + lane + 3] : Nz;
-    if (cell) atomicMin(&sh.kstart, mykmin);
+    const int own = (row + 3) * PXW + lane + 3;       // plane index of the owned column (lane < TC)
+    const int ownkm = lane < TC ? sh.km[own] : KMIN_OUTSIDE;
+    const int mykmin = cell ? ownkm : Nz;
+    // lowest active level of the tile, by every wavefront for itself
+    int low = Nz;
+    if (lane < TC && ci < g.Nx)
+#pragma unroll
+        for (int r = 0; r < TR; r++)
+            if (j0 + r < g.Ny) low = min(low, sh.km[(r + 3) * PXW + lane + 3]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) low = min(low, __shfl_xor(low, off));
+    const int klow = wave_uniform(low);
+    const int kstart = max(klow, k0);
 
     // Per-tile addressing and face thresholds (independent of the level)
-    int pkm[NPL];
     uint32_t poff[NPL];
+    int pidx[NPL];
 #pragma unroll
     for (int q = 0; q < NPL; q++) {
-        const int n = tid + q * NTHR;
-        pkm[q] = NEVER;
+        const int n = tid + q * NTHR, m = n - 6 * PXW;
+        const int r = n / PXW, c = m % 6;
+        const int pj = m < 0 ? (r < 3 ? r : r + TR) : 3 + m / 6;
+        const int pi = m < 0 ? n % PXW : (c < 3 ? c : c + TC);
+        pidx[q] = n < NH ? pj * PXW + pi : 0;
         poff[q] = 0;
-        if (n < PN) {
-            pkm[q] = sh.km[n];
-            if (pkm[q] < KMIN_OUTSIDE) {
-                const int gi = g.wx(i0 - 3 + n % PXW), gj = g.wy(j0 - 3 + n / PXW);
-                poff[q] = (uint32_t)gi * ES + (uint32_t)gj * L.c_sy;
-            }
-        }
+        if (n < NH && sh.km[pidx[q]] < KMIN_OUTSIDE)
+            poff[q] = (uint32_t)g.wx(i0 - 3 + pi) * ES + (uint32_t)g.wy(j0 - 3 + pj) * L.c_sy;
     }
     const bool xrow = cj < g.Ny;                 // this wavefront's row is inside the domain
     const bool ycol = lane < TC && ci < g.Nx;
@@ -262,13 +285,12 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
     const uint32_t uoff = xrow ? (uint32_t)fiw * ES + (uint32_t)cj * L.u_sy : 0u;
     const uint32_t voff_s = ycol ? (uint32_t)cy * ES + (uint32_t)fjs * L.v_sy : 0u;
     const uint32_t dvn = (uint32_t)(fjn - fjs) * L.v_sy;           // north face: voff_s + dvn (uniform)
-    const uint32_t coff = cell ? (uint32_t)ci * ES + (uint32_t)cj * L.c_sy : 0u;
+    // the owned column; past a periodic edge the wrapped one, which the tile's last cells read
+    const uint32_t coff = ownkm < KMIN_OUTSIDE ? (uint32_t)fiw * ES + (uint32_t)fjs * L.c_sy : 0u;
     const uint32_t dw = (uint32_t)cj * (L.w_sy - L.c_sy);           // w of the cell: coff + dw (uniform)
     auto joff = [&]() { return (uint32_t)ci * 8u + (uint32_t)cj * L.j_sy; };   // 2-D fluxes (cells only)
-    __syncthreads();
-    const int kstart = sh.kstart;
     if (MODE == 1 && cell)
-        for (int k = 0; k < mykmin && k < Nz; k++) {
+        for (int k = k0; k < mykmin && k < k1; k++) {
             stb(Tout, coff + (uint32_t)k * L.c_sz, (R)0);
             stb(Sout, coff + (uint32_t)k * L.c_sz, (R)0);
         }
@@ -282,24 +304,7 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
     constexpr bool CONS = WATCH && MODE == 0 && sizeof(R) == 4;
     const bool resid = CONS && F.residual != nullptr;   // uniform
     double resT = 0.0, resS = 0.0;
-    if (kstart >= Nz) {  // uniform: the whole tile is land
-        if (watch && cell) F.freeze_flags[(int64_t)ci + (int64_t)cj * g.Nx] = 0;
-        return;
-    }
-
-    // Vertical register window of the owned column: levels k-2 … k+3 while level k is
-    // computed; level k+3 arrives with the level's other inputs (below).
-    R zT[6], zS[6];
-#pragma unroll
-    for (int n = 0; n < 5; n++) {
-        int kk = kstart - 2 + n;
-        bool a = cell && kk >= mykmin && kk < Nz;
-        zT[n] = a ? ldb(Tin, coff + (uint32_t)kk * L.c_sz) : (R)0;
-        zS[n] = a ? ldb(Sin, coff + (uint32_t)kk * L.c_sz) : (R)0;
-    }
-    zT[5] = (R)0;
-    zS[5] = (R)0;
-    R FzT = (R)0, FzS = (R)0;  // flux through the bottom face of the current level
+    if (kstart >= k1) return;   // uniform: no active cell of the tile in the chunk
 
     // TwoColorRadiation: J₀ of the column and the surface height η of the Beer's-law factors
     const bool tc = TWO_COLOR && F.two_color != 0;   // instances without it carry none of its registers
@@ -353,22 +358,48 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
             nS0 = ldb(S0, coff + (uint32_t)k * L.c_sz);
         }
     };
+    // Vertical register window of the owned column: levels k-2 … k+3 while level k is computed;
+    // level k+3 arrives with the level's other inputs (levels outside the grid and inactive ones
+    // hold values that no face order admits).
+    R zT[6], zS[6];
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+        const uint32_t kz = (uint32_t)min(max(kstart - 2 + n, 0), Nz - 1) * L.c_sz;
+        zT[n] = ldb(Tin, coff + kz);
+        zS[n] = ldb(Sin, coff + kz);
+    }
     load_plane(kstart);
     load_u(kstart);
     load_v(kstart);
     load_w(kstart);
     load_c0(kstart);
-    for (int k = kstart; k < Nz; k++) {
-        const int kn = min(k + 1, Nz - 1);   // the level loaded ahead (the last one again at the top)
+    zT[5] = (R)0;
+    zS[5] = (R)0;
+    R FzT = (R)0, FzS = (R)0;  // flux through the bottom face of the current level
+    if (kstart > klow && adv) {   // the chunk's bottom face: between cells kstart-1 and kstart
+        const uint32_t kz = (uint32_t)max(kstart - 3, 0) * L.c_sz;
+        const R wb = ldb(w, woff_l + (uint32_t)kstart * L.w_sz);
+        const R bT = ldb(Tin, coff + kz), bS = ldb(Sin, coff + kz);
+        const int order = z_order(kstart - 1, mykmin, Nz);
+        if (cell && order > 0) {
+            FzT = (R)Azc * wb * face_value(bT, zT[0], zT[1], zT[2], zT[3], zT[4], order, wb);
+            FzS = (R)Azc * wb * face_value(bS, zS[0], zS[1], zS[2], zS[3], zS[4], order, wb);
+        }
+    }
+    for (int k = kstart; k < k1; k++) {
+        const int kn = min(k + 1, k1 - 1);   // the level loaded ahead (the last one again at the top)
         const uint32_t kc = (uint32_t)k * L.c_sz;
         // 1. stage the plane of level k; take its velocities, c⁰ and the window's top
 #pragma unroll
         for (int q = 0; q < NPL; q++) {
-            const int n = tid + q * NTHR;
-            if (n < PN) {
-                sh.cT[n] = nT[q];
-                sh.cS[n] = nS[q];
+            if (tid + q * NTHR < NH) {
+                sh.cT[pidx[q]] = nT[q];
+                sh.cS[pidx[q]] = nS[q];
             }
+        }
+        if (lane < TC) {
+            sh.cT[own] = zT[2];
+            sh.cS[own] = zS[2];
         }
         const double dzd = wave_uniform(ndz), zfb = wave_uniform(nzb), zft = wave_uniform(nzt);
         zT[5] = nzT;
@@ -418,10 +449,7 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
         }
         load_v(kn);
         // 2c. z face at the top of level k (cells k-2 … k+3 of the owned column)
-        const int zorder = (cell && adv) ? (k >= mykmin && k <= Nz - 2 ? 1 : 0) +
-                                               (k >= mykmin + 1 && k <= Nz - 3 ? 1 : 0) +
-                                               (k >= mykmin + 2 && k <= Nz - 4 ? 1 : 0)
-                                         : 0;
+        const int zorder = (cell && adv) ? z_order(k, mykmin, Nz) : 0;
         R FztT = (R)0, FztS = (R)0;
         if (zorder > 0) {
             FztT = (R)Azc * nw * face_value(zT[0], zT[1], zT[2], zT[3], zT[4], zT[5], zorder, nw);
@@ -506,8 +534,9 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
 #pragma unroll
         for (int n = 0; n < 5; n++) { zT[n] = zT[n + 1]; zS[n] = zS[n + 1]; }
     }
-    if (watch && cell) F.freeze_flags[(int64_t)ci + (int64_t)cj * g.Nx] = frz ? 1 : 0;
-    if (resid) {   // the tile's residuals: each row's by a fixed butterfly, then the rows in order
+    // set by any chunk of the column; the surface update clears a flag when it has visited the column
+    if (watch && cell && frz) F.freeze_flags[(int64_t)ci + (int64_t)cj * g.Nx] = 1;
+    if (resid) {   // the chunk's residuals: each row's by a fixed butterfly, then the rows in order
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
             resT += __shfl_xor(resT, off);
@@ -518,7 +547,7 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
             sh.resid[2 * row + 1] = resS;
         }
         __syncthreads();
-        if (tid == 0) {   // into the tile's running double-double totals
+        if (tid == 0) {   // into the chunk's running double-double totals
             double sT = 0.0, sS = 0.0;
             for (int r = 0; r < TR; r++) {
                 sT += sh.resid[2 * r];
@@ -534,25 +563,30 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
     }
 }
 
-// Single model: one block per tile, tiles ordered so that each XCD (blocks are dealt
-// round-robin to the 8 XCDs) receives a contiguous band of tiles.
+// Single model: one block per tile and chunk of levels, ordered so that each XCD (blocks are dealt
+// round-robin to the 8 XCDs) receives a contiguous band of tiles, its uppermost chunks first: they
+// hold the most active cells, and the short blocks of the lower chunks fill the launch's tail.
 template <typename Real, int MODE, bool TWO_COLOR, bool WATCH = false, bool BEER = false>
 __global__ void __launch_bounds__(TW * PLAIN_TR)
 __attribute__((amdgpu_waves_per_eu(stage_waves<Real, TWO_COLOR, WATCH && MODE == 0>())))
 tracer_tile_kernel(GridDev g, TracerLayout L, const Real* u, const Real* v, const Real* w, const Real* T0,
                    const Real* S0, const Real* Tin, const Real* Sin, Real* Tout, Real* Sout, const double* JT,
-                   const double* JS, const double* Jw, TracerForcing F, double beta_dt, int stochastic,
+                   const double* JS, const double* Jw, TracerForcing F, double beta_dt, int levels, int stochastic,
                    uint32_t seed) {
     __shared__ TileShared<Real, PLAIN_TR> sh;
     const int ntx = tiles_x(g.Nx), nty = tiles_y(g.Ny, PLAIN_TR);
+    const int nch = level_chunks(g.Nz, levels);
     const int ntiles = ntx * nty;
     const int per = (ntiles + NXCD - 1) / NXCD;
-    const int tile = (int)(blockIdx.x % NXCD) * per + (int)(blockIdx.x / NXCD);
+    const int q = (int)(blockIdx.x / NXCD) % per;
+    const int chunk = nch - 1 - (int)(blockIdx.x / NXCD) / per;
+    const int tile = (int)(blockIdx.x % NXCD) * per + q;
     if (tile >= ntiles) return;
-    if (F.residual) F.residual += RESIDUAL_SLOT * tile;   // this tile's totals
+    if (F.residual) F.residual += RESIDUAL_SLOT * (tile * nch + chunk);   // this chunk's totals
+    const int k0 = chunk * levels;
     tile_body<Real, MODE, PLAIN_TR, TWO_COLOR, WATCH, BEER>(sh, g, L, u, v, w, T0, S0, Tin, Sin, Tout, Sout, JT, JS, Jw, F,
-                                                     beta_dt, (tile % ntx) * TC, (tile / ntx) * PLAIN_TR,
-                                                     stochastic != 0, seed);
+                                                     beta_dt, (tile % ntx) * TC, (tile / ntx) * PLAIN_TR, k0,
+                                                     min(k0 + levels, g.Nz), stochastic != 0, seed);
 }
 
 // Ensemble: a persistent grid walks the (member, tile) work list. The list is cut into 8
@@ -574,7 +608,8 @@ batch_stage_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem* __re
         const BatchRec<Real>& rc = recs[it.member];
         const GridDev g = rc.g;
         const TracerLayout L = tracer_layout(rc);
-        const int ntx = tiles_x(g.Nx);
+        const int ntx = tiles_x(g.Nx), nch = level_chunks(g.Nz, rc.levels);
+        const int tile = it.index / nch, k0 = (it.index % nch) * rc.levels;
         const Real* Tin = stage == 1 ? rc.T.p : stage == 2 ? rc.T1.p : rc.T2.p;
         const Real* Sin = stage == 1 ? rc.S.p : stage == 2 ? rc.S1.p : rc.S2.p;
         Real* Tout = stage == 1 ? rc.T1.p : stage == 2 ? rc.T2.p : rc.T.p;
@@ -596,8 +631,8 @@ batch_stage_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem* __re
         }
         __syncthreads();   // the previous item's reads of the LDS are complete
         tile_body<Real, 0, TR, TWO_COLOR, WATCH, TWO_COLOR>(sh, g, L, rc.u.p, rc.v.p, rc.w.p, rc.T.p, rc.S.p, Tin, Sin, Tout, Sout, rc.n.J_T.p,
-                               rc.n.J_S.p, rc.n.J_w.p, F, beta_dt, (it.index % ntx) * TC, (it.index / ntx) * TR,
-                               stage == 3, step_seed(rc.time));
+                               rc.n.J_S.p, rc.n.J_w.p, F, beta_dt, (tile % ntx) * TC, (tile / ntx) * TR, k0,
+                               min(k0 + rc.levels, g.Nz), stage == 3, step_seed(rc.time));
     }
 }
 
@@ -837,29 +872,36 @@ hipError_t launch_rk_stage(const GridDev& g, View3<const Real> u, View3<const Re
                            View3<const double> Jw, TracerForcing forcing, double beta_dt, bool stochastic,
                            double time, hipStream_t s) {
     TracerLayout L = host_layout<Real>(Tin, u, v, w, JT);
-    const dim3 grid(grid_blocks(g.Nx, g.Ny)), block(TW, PLAIN_TR);
+    const int levels = stage_levels(g, stage_tile_levels(g));
+    const dim3 grid(grid_blocks(g, levels)), block(TW, PLAIN_TR);
     const int sr = stochastic ? 1 : 0;
     const uint32_t seed = step_seed(time);
     const bool watch = forcing.freeze_flags != nullptr;
     const bool beer = forcing.beer != nullptr;   // a model's factors (per-phase calls compute them)
     if (forcing.two_color && watch && beer)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, true, true>), grid, block, 0, s, g, L, u.p, v.p, w.p,
-                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, sr, seed);
+                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           sr, seed);
     else if (forcing.two_color && beer)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, false, true>), grid, block, 0, s, g, L, u.p, v.p, w.p,
-                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, sr, seed);
+                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           sr, seed);
     else if (forcing.two_color && watch)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, true>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, sr, seed);
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           sr, seed);
     else if (forcing.two_color)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, false>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, sr, seed);
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           sr, seed);
     else if (watch)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, false, true>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, sr, seed);
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           sr, seed);
     else
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, false, false>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, sr, seed);
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           sr, seed);
     return hipGetLastError();
 }
 template hipError_t launch_rk_stage<double>(const GridDev&, View3<const double>, View3<const double>,
@@ -916,14 +958,14 @@ hipError_t launch_tendency(const GridDev& g, View3<const Real> u, View3<const Re
                            View3<const double> JS, View3<const double> Jw, TracerForcing forcing, View3<Real> GT,
                            View3<Real> GS, hipStream_t s) {
     TracerLayout L = host_layout<Real>(T, u, v, w, JT);
+    const int levels = stage_levels(g, stage_tile_levels(g));
+    const dim3 grid(grid_blocks(g, levels)), block(TW, PLAIN_TR);
     if (forcing.two_color)
-        hipLaunchKernelGGL((tracer_tile_kernel<Real, 1, true>), dim3(grid_blocks(g.Nx, g.Ny)), dim3(TW, PLAIN_TR), 0,
-                           s, g, L, u.p, v.p, w.p, T.p, S.p, T.p, S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0, 0,
-                           0u);
+        hipLaunchKernelGGL((tracer_tile_kernel<Real, 1, true>), grid, block, 0, s, g, L, u.p, v.p, w.p, T.p, S.p, T.p,
+                           S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0, levels, 0, 0u);
     else
-        hipLaunchKernelGGL((tracer_tile_kernel<Real, 1, false>), dim3(grid_blocks(g.Nx, g.Ny)), dim3(TW, PLAIN_TR),
-                           0, s, g, L, u.p, v.p, w.p, T.p, S.p, T.p, S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0,
-                           0, 0u);
+        hipLaunchKernelGGL((tracer_tile_kernel<Real, 1, false>), grid, block, 0, s, g, L, u.p, v.p, w.p, T.p, S.p,
+                           T.p, S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0, levels, 0, 0u);
     return hipGetLastError();
 }
 template hipError_t launch_tendency<double>(const GridDev&, View3<const double>, View3<const double>,
@@ -992,10 +1034,30 @@ int64_t budget_blocks(const GridDev& g) {
 
 // The kernels of launch_budget with the partials in the device's `scratch` array; allocates
 // nothing. Every block overwrites its own pair, so nothing needs clearing between calls.
-// One slot of 4 doubles per tile of the tiling with the most tiles (the fewest rows: the
-// single-model tiling or the batch's 4-row one); a batch of taller tiles uses the first slots.
+// One slot of 4 doubles per tile and chunk of levels of the tiling with the most tiles (the fewest
+// rows: the single-model tiling or the batch's 4-row one); a batch of taller tiles uses the first
+// slots.
 int64_t residual_slots(const GridDev& g) {
-    return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR < 4 ? PLAIN_TR : 4);
+    return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR < 4 ? PLAIN_TR : 4) * level_chunks(g.Nz, stage_levels(g, stage_tile_levels(g)));
+}
+
+// Levels of one block. A block takes its levels in series, about 2.7 µs each when the chip is not
+// full, so a grid (or batch) of few tiles has each tile's column cut into chunks until there are
+// about NE_STAGE_TARGET_BLOCKS blocks; every chunk pays the tile's set-up and one more z face
+// (≈ 1.5 levels), so full grids are not cut. 1024 blocks of the FP64 kernel are resident at once;
+// 1536 measured best over 768 … 3072 (whole steps, uncut → cut, µs: one column of 50 levels
+// 166 → 57, 90×40×10 139 → 89, 353×137×19 mixed 235 → 142, 481×187×23 578 → 485, 12 uneven FP64
+// members 448 → 362 and mixed ones 295 → 122; 1440×560×10 has 3220 tiles and stays uncut: two chunks
+// per tile took its FP64 stage from 136 to 151 µs).
+#ifndef NE_STAGE_TARGET_BLOCKS
+#define NE_STAGE_TARGET_BLOCKS 1536
+#endif
+int64_t stage_tile_levels(const GridDev& g) { return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR) * g.Nz; }
+
+int stage_levels(const GridDev& g, int64_t tile_levels) {
+    const int64_t wanted = std::max<int64_t>((tile_levels + NE_STAGE_TARGET_BLOCKS - 1) / NE_STAGE_TARGET_BLOCKS, 1);
+    const int chunks = (int)((g.Nz + wanted - 1) / wanted);
+    return (g.Nz + chunks - 1) / chunks;
 }
 
 hipError_t launch_residual_reduce(const double* residual, const GridDev& g, double* out, hipStream_t s) {
