@@ -50,7 +50,7 @@ def emit(name, cs):
     through scalar_const (scalar registers at the point of use)."""
     expr = f"scalar_const((T){float(cs[-1]):.17e})"
     for c in reversed(cs[:-1]):
-        expr = f"({expr} * z + scalar_const((T){float(c):.17e}))"
+        expr = f"fma({expr}, z, scalar_const((T){float(c):.17e}))"
     return f"template <typename T>\n__device__ __forceinline__ T {name}(T z) {{\n    return {expr};\n}}\n"
 
 

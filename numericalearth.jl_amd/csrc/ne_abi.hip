@@ -4,6 +4,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
 #include <new>
 #include <vector>
 
@@ -17,6 +18,8 @@ namespace {
 inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
 inline int dev_err(hipError_t e) { return e == hipSuccess ? NE_OK : NE_ERR_DEVICE; }
+
+constexpr size_t COUNTER_BYTES = COUNTER_STRIPES * COUNTER_STRIPE_BYTES;
 
 int check_grid(const ne_grid* g) {
     if (!g) return NE_ERR_NULL;
@@ -338,8 +341,8 @@ int ne_ctx_create(int device, ne_ctx** out) {
     c->device = device;
     c->scratch = nullptr;
     c->scratch_bytes = 0;
-    if (hipMalloc((void**)&c->counters, sizeof(ne_counters)) != hipSuccess) { delete c; return NE_ERR_DEVICE; }
-    if (hipMemset(c->counters, 0, sizeof(ne_counters)) != hipSuccess ||
+    if (hipMalloc((void**)&c->counters, COUNTER_BYTES) != hipSuccess) { delete c; return NE_ERR_DEVICE; }
+    if (hipMemset(c->counters, 0, COUNTER_BYTES) != hipSuccess ||
         budget_noalloc_init(device) != hipSuccess) {   // once per device, with `device` current
         (void)hipFree(c->counters);
         delete c;
@@ -362,11 +365,24 @@ int ne_ctx_destroy(ne_ctx* c) {
 int ne_ctx_counters(ne_ctx* c, ne_counters* out, int reset, void* stream) {
     if (!c || !out) return NE_ERR_NULL;
     hipStream_t s = as_stream(stream);
-    if (hipMemcpyAsync(out, c->counters, sizeof(ne_counters), hipMemcpyDeviceToHost, s) != hipSuccess)
+    std::unique_ptr<char[]> stripes(new (std::nothrow) char[COUNTER_BYTES]);
+    if (!stripes) return NE_ERR_CAPACITY;
+    if (hipMemcpyAsync(stripes.get(), c->counters, COUNTER_BYTES, hipMemcpyDeviceToHost, s) != hipSuccess)
         return NE_ERR_DEVICE;
     if (hipStreamSynchronize(s) != hipSuccess) return NE_ERR_DEVICE;
+    ne_counters sum = {};
+    for (unsigned k = 0; k < COUNTER_STRIPES; k++) {
+        ne_counters n;
+        memcpy(&n, stripes.get() + k * COUNTER_STRIPE_BYTES, sizeof n);
+        sum.total_iterations += n.total_iterations;
+        sum.solved_columns += n.solved_columns;
+        sum.nonconverged_columns += n.nonconverged_columns;
+        sum.nan_columns += n.nan_columns;
+        sum.max_iterations = std::max(sum.max_iterations, n.max_iterations);
+    }
+    *out = sum;
     if (reset) {
-        if (hipMemsetAsync(c->counters, 0, sizeof(ne_counters), s) != hipSuccess) return NE_ERR_DEVICE;
+        if (hipMemsetAsync(c->counters, 0, COUNTER_BYTES, s) != hipSuccess) return NE_ERR_DEVICE;
         if (hipStreamSynchronize(s) != hipSuccess) return NE_ERR_DEVICE;
     }
     return NE_OK;

@@ -76,8 +76,8 @@ struct ne_batch {
     // per column-block choice: every member (finalize), and the members of each flux path (solve)
     WorkItem* surface_work[3] = {nullptr, nullptr, nullptr};
     int surface_nwork[3] = {0, 0, 0};
-    WorkItem* solve_work[3][3] = {};   // [flux path][choice]
-    int solve_nwork[3][3] = {};
+    WorkItem* solve_work[FLUX_PATHS][3] = {};   // [flux path][choice]
+    int solve_nwork[FLUX_PATHS][3] = {};
 
     ne_batch_tuning tuning;
     int cus = 256;
@@ -122,7 +122,7 @@ hipError_t enqueue_step(ne_batch* b, double dt, hipStream_t s, ne_counters* coun
     hipLaunchKernelGGL(batch_clock_kernel<Real>, dim3((n + 63) / 64), dim3(64), 0, s,
                        static_cast<BatchRec<Real>*>(b->recs), n, dt);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    for (int path = 2; path >= 0; path--) {
+    for (int path = FLUX_PATHS - 1; path >= 0; path--) {
         int nw = b->solve_nwork[path][si];
         e = launch_batch_surface_solve<Real>(recs, b->solve_work[path][si], nw, t.surface_block,
                                              std::min(blocks_for(t.surface_blocks, nw), std::max(nw, 1)), path,
@@ -185,10 +185,10 @@ BatchRec<Real> member_record(const ne_model* m, const double* atimes_dev, const 
     return r;
 }
 
-// Host-side layout of the arena: records | times | 2×3 stage lists | 3 surface lists | 3×3 solve lists.
+// Host-side layout of the arena: records | times | 2×3 stage lists | 3 surface lists | 4×3 solve lists.
 struct Layout {
     size_t recs = 0, times = 0, stage[2][3] = {{0, 0, 0}, {0, 0, 0}}, surface[3] = {0, 0, 0},
-           solve[3][3] = {};
+           solve[FLUX_PATHS][3] = {};
     size_t total = 0;
 };
 
@@ -196,7 +196,7 @@ template <typename Real>
 int rebuild(ne_batch* b, hipStream_t s) {
     const int n = (int)b->members.size();
     // work lists and snapshot times on the host
-    std::vector<WorkItem> stage[2][3], surface[3], solve[3][3];
+    std::vector<WorkItem> stage[2][3], surface[3], solve[FLUX_PATHS][3];
     std::vector<int> below_top[2][3];   // chunks above each stage item's in its tile
     std::vector<double> times;
     std::vector<size_t> aoff(n), roff(n);
@@ -254,7 +254,7 @@ int rebuild(ne_batch* b, hipStream_t s) {
         }
         L.surface[c] = off;
         off = align256(off + surface[c].size() * sizeof(WorkItem));
-        for (int f = 0; f < 3; f++) {
+        for (int f = 0; f < FLUX_PATHS; f++) {
             L.solve[f][c] = off;
             off = align256(off + solve[f][c].size() * sizeof(WorkItem));
         }
@@ -303,7 +303,7 @@ int rebuild(ne_batch* b, hipStream_t s) {
     for (int c = 0; c < 3; c++) {
         for (int f = 0; f < 2; f++) put(L.stage[f][c], stage[f][c], &b->stage_work[f][c], &b->stage_nwork[f][c]);
         put(L.surface[c], surface[c], &b->surface_work[c], &b->surface_nwork[c]);
-        for (int f = 0; f < 3; f++) put(L.solve[f][c], solve[f][c], &b->solve_work[f][c], &b->solve_nwork[f][c]);
+        for (int f = 0; f < FLUX_PATHS; f++) put(L.solve[f][c], solve[f][c], &b->solve_work[f][c], &b->solve_nwork[f][c]);
     }
     b->recs = D + L.recs;
     if (hipMemcpyAsync(D, H, L.total, hipMemcpyHostToDevice, s) != hipSuccess) return NE_ERR_DEVICE;
@@ -407,7 +407,7 @@ int autotune(ne_batch* b, hipStream_t s, ne_batch_tuning* out) {
             double ms;
             auto f = [&]() {
                 hipError_t e = hipSuccess;
-                for (int path = 2; path >= 0 && e == hipSuccess; path--) {
+                for (int path = FLUX_PATHS - 1; path >= 0 && e == hipSuccess; path--) {
                     int nw = b->solve_nwork[path][c];
                     e = launch_batch_surface_solve<Real>(recs, b->solve_work[path][c], nw, SURFACE_BLOCKS[c],
                                                          std::min(blocks_for(req, nw), std::max(nw, 1)), path,

@@ -4,12 +4,12 @@
 // is compiled with -ffp-contract=off. The general FP64 flux instance keeps the reference's
 // evaluation order with the math library's elementary functions, apart from the saturation
 // vapour pressure (one exponential of a sum, with ne_log, for a power times an exponential,
-// within a few ulp). The instance for the default
-// Edson constants ("Fast", and "Consts" with the default surface constants as literals) departs
-// from it at the ulp level: its own logarithm ne_log, arctangent ne_atan_ge1, cube root
-// ne_cbrt_ge1, square root ne_sqrt and exponential ne_exp (each within 2 ulp), A·exp(−b·log R★) for A/R★^b, x·√x for (1 + x)^{3/2}, shared subexpressions of ψ_m and
-// ψ_s, and a degree-7 Taylor polynomial of ψ at |ζ| ≤ 5·10⁻⁴; with the default surface constants
-// also logarithms of quotients as differences of logarithms, ζ as products with 1/L, and its
+// within a few ulp). The instances for the default
+// Edson constants (flux paths 1 to 3, flux_path) depart from it at the ulp level: ψ_m and ψ_s from a
+// table of piecewise polynomials (PsiTable) and at |ζ| ≤ 5·10⁻⁴ their degree-7 Taylor polynomials,
+// A·exp(−b·log R★) for A/R★^b, and the library's own logarithm, cube root, square root and
+// exponential (each within 2 ulp); with positive surface constants (paths 2 and 3)
+// also logarithms of quotients as differences of logarithms, ζ as products with 1/L, and the
 // remaining quotients as products with a reciprocal refined by two Newton steps (quotient).
 // Those differences stay far inside the 1e-12 comparison with
 // the oracle, but near a stop threshold they can move a column's fixed point by one iteration
@@ -17,6 +17,8 @@
 // reconstructions use fused multiply-adds and a reciprocal-based division (stated there).
 #pragma once
 #include <string.h>
+
+#include <type_traits>
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -285,6 +287,7 @@ __device__ __forceinline__ double psi_scalar(const ne_params& p, double z) {
 
 #include "ne_psi_series.h"
 #include "ne_atan_poly.h"
+#include "ne_psi_table.h"
 #define NE_PSI_SERIES_RADIUS 5e-4
 
 // Elementary functions by precision: FP64 uses the math library (the Fast flux instance its
@@ -394,40 +397,124 @@ __device__ __forceinline__ T tdiv(T a, T b) { return quotient(a, b); }
 template <>
 __device__ __forceinline__ float tdiv<float>(float a, float b) { return a * frcp(b); }
 
+// ψ_m and ψ_s with the default constants as piecewise polynomials (ne_psi_table.h): intervals of
+// an eighth of a binade in t = a − ζ (ζ < 0) and t = ζ + 3/2, the distances to the functions'
+// nearest singularities, so an interval's index is the exponent and the three leading mantissa bits
+// of t, and one polynomial of degree 9 (FP64) or 4 (FP32) in t minus the interval's centre holds
+// each function to 2⁻⁵⁴ (2⁻²⁵) of max(1, |ψ|). A block copies the table to LDS (21 KB, FP32 6 KB) and
+// its work-items gather their interval's coefficients, ψ_m's and ψ_s's of a power side by side. The
+// closed forms below (psi_pair_default) take about 310 vector instructions of an iteration in FP64
+// (four logarithms, three arctangents, two cube and two square roots), this about 45: with it, the
+// logarithm below and plain selects for the iteration's minima and maxima an iteration takes about 270
+// instructions instead of 680, and the FP64 K1 of 1440×560×10 went from 295 to 188 µs (the mixed one,
+// whose FP32 functions are cheap, from 114 to 105). ζ beyond the table (below −128, above 14.5, NaN)
+// takes the closed forms; out of line, they cost more in spills around the call (195 µs).
+constexpr double PSI_A = 1.0 / 34.15;   // unstable t = PSI_A − ζ
+constexpr double PSI_B = 1.5;           // stable t = ζ + PSI_B
+
 template <typename T>
-__device__ __forceinline__ T psi_m_default(T z) {
+struct PsiTable;
+template <>
+struct PsiTable<double> {
+    double2 c[NE_PSI_BINS * 10];
+    double2 log[64];   // ne_log_table
+};
+template <>
+struct PsiTable<float> {
+    float4 c[NE_PSI_BINS * 3];
+};
+struct NoTable {};
+// The table of an FP64 iteration: none where it only finishes what an FP32 one did not.
+template <bool Mixed, typename Tab>
+__device__ __forceinline__ std::conditional_t<Mixed, NoTable, const Tab&> table64(const Tab& tab) {
+    if constexpr (Mixed) return NoTable{};
+    else return tab;
+}
+
+__device__ __forceinline__ void psi_pair(const NoTable&, double z, double& pm, double& ps);
+
+// Interval of t, counted from the unstable side's first one; out of the table: −1.
+__device__ __forceinline__ int psi_bin(bool unstable, int exponent_and_bits) {
+    const int bin = exponent_and_bits - (unstable ? (1017 << 3) + 6 : (1023 << 3) + 4 - NE_PSI_UNSTABLE_BINS);
+    return bin < (unstable ? NE_PSI_UNSTABLE_BINS : NE_PSI_BINS) ? bin : -1;
+}
+
+template <typename T>
+__device__ __forceinline__ void psi_pair_default(T z, T& pm, T& ps);
+
+__device__ __forceinline__ void psi_pair(const PsiTable<double>& tab, double z, double& pm, double& ps) {
+    const bool unstable = z < 0.0;
+    const double t = fabs(z) + (unstable ? PSI_A : PSI_B);
+    const int hi = __double2hiint(t);
+    const int bin = psi_bin(unstable, hi >> 17);
+    if (bin >= 0) {
+        const double x = t - __hiloint2double((hi & ~0x1ffff) | 0x10000, 0);
+        const double2* c = &tab.c[bin * 10];
+        double m = c[9].x, s = c[9].y;
+#pragma unroll
+        for (int n = 8; n >= 0; n--) {
+            m = fma(m, x, c[n].x);
+            s = fma(s, x, c[n].y);
+        }
+        pm = m;
+        ps = s;
+    } else {
+        psi_pair_default(z, pm, ps);
+    }
+}
+
+__device__ __forceinline__ void psi_pair(const PsiTable<float>& tab, float z, float& pm, float& ps) {
+    const bool unstable = z < 0.0f;
+    const float t = fabsf(z) + (unstable ? (float)PSI_A : (float)PSI_B);
+    const int bits = __float_as_int(t);
+    const int bin = psi_bin(unstable, (bits >> 20) + ((1023 - 127) << 3));
+    if (bin >= 0) {
+        const float x = t - __int_as_float((bits & ~0xfffff) | 0x80000);
+        const float4 a = tab.c[bin * 3], b = tab.c[bin * 3 + 1], d = tab.c[bin * 3 + 2];
+        pm = fmaf(fmaf(fmaf(fmaf(d.x, x, b.z), x, b.x), x, a.z), x, a.x);
+        ps = fmaf(fmaf(fmaf(fmaf(d.y, x, b.w), x, b.y), x, a.w), x, a.y);
+    } else {
+        psi_pair_default(z, pm, ps);
+    }
+}
+
+// ψ at ℓ/L, almost always within the series' radius.
+template <typename Tab, typename T>
+__device__ __forceinline__ T psi_m_near(const Tab& tab, T z) {
     if (fabs(z) <= (T)NE_PSI_SERIES_RADIUS) return z < (T)0 ? psi_series_momentum_unstable(z) : psi_series_momentum_stable(z);
-    const T pi = (T)3.14159265358979323846, s3 = (T)1.7320508075688772935;
-    if (z < (T)0) {
-        T xs = tsqrt((T)1 - (T)15 * z), xm = tsqrt(xs);
-        T psi1 = (T)2 * tlog(((T)1 + xm) * (T)0.5) + tlog(((T)1 + xs) * (T)0.5) - (T)2 * tatan_ge1(xm) + pi / (T)2;
-        T f2 = tcbrt_ge1((T)1 - (T)10.15 * z);
-        T psi2 = (T)1.5 * tlog(((T)1 + f2 + f2 * f2) * (T)(1.0 / 3.0)) - s3 * tatan_ge1(((T)1 + (T)2 * f2) * ((T)1 / s3)) + pi / s3;
-        T f = tdiv(z * z, (T)1 + z * z);
-        return ((T)1 - f) * psi1 + f * psi2;
-    }
-    T e = texp(-fmin((T)50, (T)0.35 * z));
-    return (T)-0.7 * z - (T)0.75 * (z - (T)(5.0 / 0.35)) * e - (T)(0.75 * (5.0 / 0.35));
+    T pm, ps;
+    psi_pair(tab, z, pm, ps);
+    return pm;
 }
-
-template <typename T>
-__device__ __forceinline__ T psi_s_default(T z) {
+template <typename Tab, typename T>
+__device__ __forceinline__ T psi_s_near(const Tab& tab, T z) {
     if (fabs(z) <= (T)NE_PSI_SERIES_RADIUS) return z < (T)0 ? psi_series_scalar_unstable(z) : psi_series_scalar_stable(z);
-    const T pi = (T)3.14159265358979323846, s3 = (T)1.7320508075688772935;
-    if (z < (T)0) {
-        T xs = tsqrt((T)1 - (T)15 * z);
-        T psi1 = (T)2 * tlog(((T)1 + xs) * (T)0.5);
-        T f2 = tcbrt_ge1((T)1 - (T)34.15 * z);
-        T psi2 = (T)1.5 * tlog(((T)1 + f2 + f2 * f2) * (T)(1.0 / 3.0)) - s3 * tatan_ge1(((T)1 + (T)2 * f2) * ((T)1 / s3)) + pi / s3;
-        T f = tdiv(z * z, (T)1 + z * z);
-        return ((T)1 - f) * psi1 + f * psi2;
-    }
-    T e = texp(-fmin((T)50, (T)0.35 * z));
-    T x = (T)1 + (T)(2.0 / 3.0) * z;
-    return -(x * tsqrt(x)) - (T)(2.0 / 3.0) * (z - (T)14.28) * e - (T)8.525;
+    T pm, ps;
+    psi_pair(tab, z, pm, ps);
+    return ps;
 }
 
-// ψ_m(ζ) and ψ_s(ζ) together (the height term h/L of the two profiles).
+// The flux iteration's logarithm with a table: x = 2^e·m, m ∈ [½, 1), 1/c and −log c of m's 64th
+// of the interval from LDS, and log1p of r = m/c − 1, |r| < 0.01, by its series to r⁷ (remainder
+// 10⁻¹⁷): 16 vector instructions where ne_log, which divides, takes 30. The error is absolute, about
+// an ulp of e·ln 2 or of 0.7, which suits sums of logarithms of size 1 to 12; next to x = 1 ne_log
+// is the accurate one.
+__device__ __forceinline__ double tlog(const PsiTable<double>& tab, double x) {
+    const double m = __builtin_amdgcn_frexp_mant(x);
+    const double de = (double)__builtin_amdgcn_frexp_exp(x);
+    const double2 c = tab.log[(__double2hiint(m) >> 14) & 63];
+    const double r = fma(m, c.x, -1.0);
+    double q = fma(1.0 / 7.0, r, -1.0 / 6.0);
+    q = fma(q, r, 1.0 / 5.0);
+    q = fma(q, r, -1.0 / 4.0);
+    q = fma(q, r, 1.0 / 3.0);
+    q = fma(q, r, -0.5);
+    const double p = fma(r * r, q, r);
+    return fma(de, 0.6931471805599453, c.y) + fma(de, 2.3190468138462996e-17, p);
+}
+__device__ __forceinline__ double tlog(const NoTable&, double x) { return ne_log(x); }
+
+// ψ_m(ζ) and ψ_s(ζ) in closed form.
 template <typename T>
 __device__ __forceinline__ void psi_pair_default(T z, T& pm, T& ps) {
     if (fabs(z) <= (T)NE_PSI_SERIES_RADIUS) {
@@ -454,6 +541,10 @@ __device__ __forceinline__ void psi_pair_default(T z, T& pm, T& ps) {
     pm = (T)-0.7 * z - (T)0.75 * (z - (T)(5.0 / 0.35)) * e - (T)(0.75 * (5.0 / 0.35));
     T x = (T)1 + (T)(2.0 / 3.0) * z;
     ps = -(x * tsqrt(x)) - (T)(2.0 / 3.0) * (z - (T)14.28) * e - (T)8.525;
+}
+
+__device__ __forceinline__ void psi_pair(const NoTable&, double z, double& pm, double& ps) {
+    psi_pair_default(z, pm, ps);
 }
 
 // True when the flux formulation is SimilarityTheoryFluxes with BulkTemperature and the
@@ -529,11 +620,31 @@ __host__ inline bool default_surface_constants(const ne_params& p) {
     return memcmp(&q, &p, sizeof q) == 0;
 }
 
-// Flux-solve instance of a parameter set: 0 the general path, 1 the reference's default
-// Edson constants (shared ψ), 2 those and the default surface constants compiled in.
+// True when the iteration may take the logarithm of every quantity it forms (flux path 3): the
+// Edson roughness lengths with positive constants, and a gustiness that keeps u★ above zero.
+__host__ inline bool positive_surface_constants(const ne_params& p) {
+    const double positive[] = {p.von_karman_constant, p.minimum_gustiness, p.roughness_gravitational_acceleration,
+                               p.air_kinematic_viscosity, p.charnock_parameter + p.smooth_wall_parameter,
+                               p.maximum_momentum_roughness, p.reynolds_scaling_A, p.maximum_scalar_roughness,
+                               p.surface_layer_height - p.zero_plane_displacement};
+    for (double x : positive)
+        if (!(x >= 1e-30 && x <= 1e30)) return false;
+    const double zero_or_positive[] = {p.gustiness_parameter, p.charnock_parameter, p.smooth_wall_parameter,
+                                       p.boundary_layer_height, fabs(p.reynolds_scaling_b)};
+    for (double x : zero_or_positive)
+        if (!(x >= 0.0 && x <= 1e30)) return false;
+    return p.convective_gustiness && p.momentum_roughness == NE_ROUGHNESS_EDSON &&
+           p.temperature_roughness == NE_ROUGHNESS_EDSON && p.water_vapor_roughness == NE_ROUGHNESS_EDSON;
+}
+
+// Flux-solve instance of a parameter set: 0 the general path, 1 the reference's default Edson
+// constants (shared ψ), 3 those and positive surface constants (the iteration in logarithms), 2 the
+// default surface constants, compiled in.
+constexpr int FLUX_PATHS = 4;
 __host__ inline int flux_path(const ne_params& p) {
     if (!edson_default_constants(p)) return 0;
-    return default_surface_constants(p) ? 2 : 1;
+    if (default_surface_constants(p)) return 2;
+    return positive_surface_constants(p) ? 3 : 1;
 }
 
 // similarity_profile (similarity_theory_turbulent_fluxes.jl:242-253)
@@ -789,6 +900,18 @@ __device__ __noinline__ int flux_iterate_general(const ne_params& p, double ua, 
 // gives them the same values. Finishing in FP64 as well (≈ 3 more FP64 iterations)
 // changed neither the 200-step SST error against the FP64 model (9.8e-6 of the largest SST)
 // nor the flux errors (2.4e-5 of their scale) at 1440×560×10, and cost 13 % of the step.
+// Latent heat, sensible heat and water vapour fluxes from the scales; returns the air density.
+__device__ __forceinline__ double scalar_fluxes(const ne_params& p, double Ta, double pa, double qa, double us,
+                                                double ts, double qs, double& Qv, double& Qt, double& Jv) {
+    const double rho = air_density(p, Ta, pa, qa);
+    const double cpm = cp_m(p, qa);
+    const double Lv = latent_heat_vapor(p, Ta);
+    Qv = -rho * Lv * us * qs;
+    Qt = -rho * cpm * us * ts;
+    Jv = -rho * us * qs;
+    return rho;
+}
+
 #ifndef NE_MIXED_DRIFT
 #define NE_MIXED_DRIFT 2e-7f
 #endif
@@ -796,11 +919,13 @@ __device__ __noinline__ int flux_iterate_general(const ne_params& p, double ua, 
 #define NE_MIXED_MAXITER 40
 #endif
 
-template <bool Fast, bool Mixed = false, bool Consts = false, bool Defer = false>
-__device__ __forceinline__ ColumnFluxes flux_column(const ne_params& p_in, double ua, double va, double Ta,
+template <int PATH, bool Mixed, bool Defer, typename Tab>
+__device__ __forceinline__ ColumnFluxes flux_column(const Tab& tab, const ne_params& p_in, double ua, double va, double Ta,
                                                     double pa, double qa, double To_C, double uo, double vo,
                                                     bool inactive, double SW = 0.0, double LW = 0.0) {
-    // Consts: the default surface constants as literals (the host has checked that p holds them)
+    constexpr bool Fast = PATH >= 1;      // default Edson constants
+    constexpr bool LogForm = PATH >= 2;   // and positive surface constants
+    constexpr bool Consts = PATH == 2;    // the default surface constants as literals (checked by the host)
     ne_params pc;
     if constexpr (Consts) {
         pc = p_in;
@@ -844,23 +969,27 @@ __device__ __forceinline__ ColumnFluxes flux_column(const ne_params& p_in, doubl
                                     p.temperature_roughness_length == p.water_vapor_roughness_length);
         const int maxit = p.maxiter;
         const double tol = p.tolerance;
-        // LogForm (the default constants compiled in): the logarithms of the profiles' quotients
+        // LogForm: the logarithms of the profiles' quotients
         // as differences of logarithms, log(h/ℓ) = log h − log ℓ, with log R★ = log ℓᵤ + log u★ −
         // log ν and log ℓq = min(log A − b·log R★, log ℓmax), so an iteration takes two
         // logarithms (ℓᵤ, u★) and no quotients where it took three of each, and the three
         // stability arguments as products with 1/L. The terms are of size ≤ 12 and the results
         // agree with the quotient forms to a few ulp of those terms. u★ > 0 (the iteration's first
         // guess, and κU over a positive profile with U ≥ the minimum gustiness).
-        constexpr bool LogForm = Fast && Consts;
         const double zd = za - p.zero_plane_displacement;
-        const double ln_nu = LogForm ? ne_log(p.air_kinematic_viscosity) : 0.0;
-        const double ln_A = LogForm ? ne_log(p.reynolds_scaling_A) : 0.0;
-        const double ln_lqmax = LogForm ? ne_log(p.maximum_scalar_roughness) : 0.0;
-        const double ln_zd = LogForm ? ne_log(zd) : 0.0;
+        // (the compiler evaluates the logarithms of literals)
+        auto constant_log = [](double x) { return Consts ? __builtin_log(x) : ne_log(x); };
+        const double ln_nu = LogForm ? constant_log(p.air_kinematic_viscosity) : 0.0;
+        const double ln_A = LogForm ? constant_log(p.reynolds_scaling_A) : 0.0;
+        const double ln_lqmax = LogForm ? constant_log(p.maximum_scalar_roughness) : 0.0;
+        const double ln_zd = LogForm ? constant_log(zd) : 0.0;
         const double ln2 = 0.6931471805599453;
+        const double Cg_g = p.charnock_parameter / p.roughness_gravitational_acceleration;
+        const double Cnu_nu = p.smooth_wall_parameter * p.air_kinematic_viscosity;
 
         bool done32 = false;   // the FP32 fixed point converged: no FP64 iteration
-        if (Mixed && Fast && converge && shared_scalar && p.momentum_roughness == NE_ROUGHNESS_EDSON &&
+        if constexpr (Mixed && Fast)
+        if (converge && shared_scalar && p.momentum_roughness == NE_ROUGHNESS_EDSON &&
             p.water_vapor_roughness == NE_ROUGHNESS_EDSON) {
             const float fgoTv = (float)goTv, fonedq = (float)onedq, fdTv = (float)dTv;
             const float fdu2dv2 = (float)du2dv2, fdtheta = (float)dtheta, fdq = (float)dq;
@@ -890,9 +1019,9 @@ __device__ __forceinline__ ColumnFluxes flux_column(const ne_params& p_in, doubl
                 float dh = fmaxf(fzd, 2.0f * lu);
                 float L = bstar == 0.0f ? (float)INFINITY : tdiv(fus * fus, fkappa * bstar);
                 float pmh, psh;
-                psi_pair_default<float>(tdiv(dh, L), pmh, psh);
-                float chiu = tdiv(fkappa, tlog(tdiv(dh, lu)) - pmh + psi_m_default<float>(tdiv(lu, L)));
-                float chiq = tdiv(fkappa, tlog(tdiv(dh, lq)) - psh + psi_s_default<float>(tdiv(lq, L)));
+                psi_pair(tab, tdiv(dh, L), pmh, psh);
+                float chiu = tdiv(fkappa, tlog(tdiv(dh, lu)) - pmh + psi_m_near(tab, tdiv(lu, L)));
+                float chiq = tdiv(fkappa, tlog(tdiv(dh, lq)) - psh + psi_s_near(tab, tdiv(lq, L)));
                 float nus = chiu * U, nts = chiq * fdtheta, nqs = chiq * fdq;
                 float drift = fabsf(nus - fus) + fabsf(nts - fts) + fabsf(nqs - fqs);
                 fus = nus; fts = nts; fqs = nqs;
@@ -922,12 +1051,16 @@ __device__ __forceinline__ ColumnFluxes flux_column(const ne_params& p_in, doubl
             double bstar = goTv * (ts * onedq + dTv * qs);
             double Usg2;
             if constexpr (LogForm) {
-                // the default convective gustiness with ne_cbrt_ge1's first value and Halley step,
-                // valid for any x in FP32's normal range: below 10⁻³⁰, β∛x is far under the
-                // minimum gustiness the maximum keeps, so x is taken as 0 there
-                const double x = jmax(0.0, -us * bstar) * hbl;
-                const double Ug = jmax(p.minimum_gustiness, p.gustiness_parameter * (x < 1e-30 ? 0.0 : ne_cbrt_ge1(x)));
+                // the convective gustiness with ne_cbrt_ge1's first value and Halley step, valid for
+                // any x in FP32's normal range: below 10⁻³⁰, β∛x is far under the minimum
+                // gustiness the maximum keeps, so x is taken as 0 there. Minima and maxima are plain
+                // selects here: a NaN of the iterate reaches all three scales through u★ or 1/L
+                const double Jb = -us * bstar;
+                const double x = (Jb > 0.0 ? Jb : 0.0) * hbl;
+                const double w = p.gustiness_parameter * (x < 1e-30 ? 0.0 : ne_cbrt_ge1(x));
+                const double Ug = w > p.minimum_gustiness ? w : p.minimum_gustiness;
                 Usg2 = Ug * Ug;
+                if (p.mesoscale_gustiness) Usg2 = Usg2 + p.mesoscale_velocity * p.mesoscale_velocity;
             } else {
                 Usg2 = gustiness_squared(p, us, bstar, hbl);
             }
@@ -935,42 +1068,45 @@ __device__ __forceinline__ ColumnFluxes flux_column(const ne_params& p_in, doubl
             // LogForm: 1/u★ once (hardware reciprocal and two Newton steps), for ℓᵤ's smooth-wall
             // term and for 1/L; the Charnock term with Cg/g folded
             const double rus = LogForm ? quotient(1.0, us) : 0.0;
-            double lu = LogForm ? jmin((p.charnock_parameter / p.roughness_gravitational_acceleration) * (us * us) +
-                                           (p.smooth_wall_parameter * p.air_kinematic_viscosity) * rus,
-                                       p.maximum_momentum_roughness)
-                                : momentum_roughness(p, us);
-            double lq, lt, lnlu = 0.0, lnlq = 0.0;
+            double lu, lq, lt, lnlu = 0.0, lnlq = 0.0;
             if constexpr (LogForm) {
-                lnlu = ne_log(lu);
-                const double lnRs = lnlu + ne_log(us) - ln_nu;
-                lq = jmin(p.reynolds_scaling_A * ne_exp(-p.reynolds_scaling_b * lnRs), p.maximum_scalar_roughness);
-                lnlq = jmin(ln_A - p.reynolds_scaling_b * lnRs, ln_lqmax);
+                lu = Cg_g * (us * us) + Cnu_nu * rus;
+                lu = lu < p.maximum_momentum_roughness ? lu : p.maximum_momentum_roughness;
+                lnlu = tlog(table64<Mixed>(tab), lu);
+                const double lnRs = lnlu + tlog(table64<Mixed>(tab), us) - ln_nu;
+                lq = p.reynolds_scaling_A * ne_exp(-p.reynolds_scaling_b * lnRs);
+                lq = lq < p.maximum_scalar_roughness ? lq : p.maximum_scalar_roughness;
+                lnlq = ln_A - p.reynolds_scaling_b * lnRs;
+                lnlq = lnlq < ln_lqmax ? lnlq : ln_lqmax;
             } else if (Fast && p.water_vapor_roughness == NE_ROUGHNESS_EDSON) {
+                lu = momentum_roughness(p, us);
                 double Rstar = lu * us / p.air_kinematic_viscosity;
                 double ls = Rstar == 0.0 ? 0.0 : p.reynolds_scaling_A * exp(-p.reynolds_scaling_b * ne_log(Rstar));
                 lq = jmin(ls, p.maximum_scalar_roughness);
             } else {
+                lu = momentum_roughness(p, us);
                 lq = scalar_roughness(p, p.water_vapor_roughness, p.water_vapor_roughness_length, lu, us);
             }
             lt = shared_scalar ? lq
                                : scalar_roughness(p, p.temperature_roughness, p.temperature_roughness_length, lu, us);
-            double dh = jmax(za - p.zero_plane_displacement, 2.0 * lu);
+            const double dh = LogForm ? (2.0 * lu > zd ? 2.0 * lu : zd) : jmax(zd, 2.0 * lu);
             double chiu, chiq, chit;
             if constexpr (LogForm) {
                 const double invL = (kappa * bstar) * (rus * rus);
                 const double lndh = 2.0 * lu > zd ? ln2 + lnlu : ln_zd;
                 double pmh, psh;
-                psi_pair_default(dh * invL, pmh, psh);
-                chiu = quotient(kappa, (lndh - lnlu) - pmh + psi_m_default(lu * invL));
-                chiq = quotient(kappa, (lndh - lnlq) - psh + psi_s_default(lq * invL));
+                psi_pair(table64<Mixed>(tab), dh * invL, pmh, psh);
+                chiu = quotient(kappa, (lndh - lnlu) - pmh + psi_m_near(table64<Mixed>(tab), lu * invL));
+                chiq = quotient(kappa, (lndh - lnlq) - psh + psi_s_near(table64<Mixed>(tab), lq * invL));
                 chit = chiq;
-            } else if (Fast) {
+            } else if constexpr (Fast) {
                 double L = bstar == 0.0 ? (double)INFINITY : us * us / (kappa * bstar);
                 double pmh, psh;
-                psi_pair_default(dh / L, pmh, psh);
-                chiu = kappa / (ne_log(dh / lu) - pmh + psi_m_default(lu / L));
-                chiq = kappa / (ne_log(dh / lq) - psh + psi_s_default(lq / L));
-                chit = shared_scalar ? chiq : kappa / (ne_log(dh / lt) - psh + psi_s_default(lt / L));
+                psi_pair(table64<Mixed>(tab), dh / L, pmh, psh);
+                chiu = kappa / (ne_log(dh / lu) - pmh + psi_m_near(table64<Mixed>(tab), lu / L));
+                chiq = kappa / (ne_log(dh / lq) - psh + psi_s_near(table64<Mixed>(tab), lq / L));
+                chit = shared_scalar ? chiq
+                                     : kappa / (ne_log(dh / lt) - psh + psi_s_near(table64<Mixed>(tab), lt / L));
             } else {
                 double L = bstar == 0.0 ? (double)INFINITY : us * us / (kappa * bstar);
                 chiu = kappa / similarity_profile(p, false, dh, lu, L);
@@ -1004,13 +1140,8 @@ __device__ __forceinline__ ColumnFluxes flux_column(const ne_params& p_in, doubl
     double dU = sqrt(du * du + dv * dv);
     double taux = dU == 0.0 ? 0.0 : -(us * us) * du / dU;
     double tauy = dU == 0.0 ? 0.0 : -(us * us) * dv / dU;
-    double rho = air_density(p, Ta, pa, qa);
-    double cpm = cp_m(p, qa);
-    double Lv = latent_heat_vapor(p, Ta);
     ColumnFluxes r;
-    r.Qv = -rho * Lv * us * qs;
-    r.Qt = -rho * cpm * us * ts;
-    r.Jv = -rho * us * qs;
+    const double rho = scalar_fluxes(p, Ta, pa, qa, us, ts, qs, r.Qv, r.Qt, r.Jv);
     r.rtx = rho * taux;
     r.rty = rho * tauy;
     r.us = us;

@@ -7,9 +7,14 @@
 
 #include "ne_device.h"
 
+// Copies of the solver counters of a context (ne_surface.hip: counter_stripe), a cache line each.
+constexpr unsigned COUNTER_STRIPES = 1024;
+constexpr size_t COUNTER_STRIPE_BYTES = 128;
+static_assert(sizeof(ne_counters) <= COUNTER_STRIPE_BYTES, "a stripe holds the counters");
+
 struct ne_ctx {
     int device;
-    ne_counters* counters;      // device
+    ne_counters* counters;      // device, COUNTER_STRIPES copies of COUNTER_STRIPE_BYTES each
     double* scratch;            // device workspace (budget partials), grown on demand
     size_t scratch_bytes;
 };
@@ -264,7 +269,7 @@ struct BatchRec {
     int nat, nrt;
     int time_indexing;      // NE_TIME_CLAMPED or NE_TIME_CYCLICAL
     double time_period;
-    int fast;               // flux path (flux_path): 0 general, 1 default Edson constants, 2 also default constants
+    int fast;               // flux path (flux_path)
     double time;           // device clock of the member (advanced by the clock kernel)
 };
 

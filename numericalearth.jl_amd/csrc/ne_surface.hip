@@ -73,90 +73,51 @@ __device__ __forceinline__ int solve_order_key(const FluxOut& out, int i, int j)
     return stable ? SORT_BINS / 2 - 1 + it : it;
 }
 
-// Block-wide reduction of the solver counters, then one atomic per block (blocks of a
-// power-of-two number of work-items, at most N).
-template <int N = BX * BY>
-__device__ void accumulate_counters(ne_counters* c, bool solved, int it, bool nonconv, bool nan) {
-    __shared__ unsigned s_it[N], s_solved[N], s_nc[N], s_nan[N], s_max[N];
-    int t = threadIdx.x + threadIdx.y * blockDim.x;
-    int n = blockDim.x * blockDim.y;
-    s_it[t] = solved ? (unsigned)it : 0u;
-    s_solved[t] = solved ? 1u : 0u;
-    s_nc[t] = (solved && nonconv) ? 1u : 0u;
-    s_nan[t] = (solved && nan) ? 1u : 0u;
-    s_max[t] = solved ? (unsigned)it : 0u;
-    __syncthreads();
-    for (int w = n / 2; w > 0; w >>= 1) {
-        if (t < w) {
-            s_it[t] += s_it[t + w];
-            s_solved[t] += s_solved[t + w];
-            s_nc[t] += s_nc[t + w];
-            s_nan[t] += s_nan[t + w];
-            s_max[t] = s_max[t] > s_max[t + w] ? s_max[t] : s_max[t + w];
-        }
-        __syncthreads();
-    }
-    if (t == 0 && c != nullptr && s_solved[0] > 0) {
-        atomicAdd((unsigned long long*)&c->total_iterations, (unsigned long long)s_it[0]);
-        atomicAdd(&c->solved_columns, s_solved[0]);
-        if (s_nc[0]) atomicAdd(&c->nonconverged_columns, s_nc[0]);
-        if (s_nan[0]) atomicAdd(&c->nan_columns, s_nan[0]);
-        atomicMax(&c->max_iterations, s_max[0]);
-    }
+// The solver counters are kept in COUNTER_STRIPES copies, each in a cache line of its own and summed
+// when they are read; a wavefront adds to the copy of its number, so that few share an address, and
+// waits for no other wavefront. With one copy, to which 3150 blocks added after a reduction over the
+// block, the counters took 28 µs of the 1440×560×10 FP64 K1 and 30 µs of the mixed one's 93: all
+// XCDs' atomics queued on one line of memory, and the block's wavefronts waited for its slowest.
+__device__ __forceinline__ ne_counters* counter_stripe(ne_counters* c) {
+    const unsigned t = threadIdx.x + threadIdx.y * blockDim.x, waves = (blockDim.x * blockDim.y + 63) / 64;
+    const unsigned w = (blockIdx.x + blockIdx.y * gridDim.x) * waves + (t >> 6);
+    return reinterpret_cast<ne_counters*>(reinterpret_cast<char*>(c) + (w % COUNTER_STRIPES) * COUNTER_STRIPE_BYTES);
 }
 
-// The solver counters of a block, added once at the kernel's end from per-work-item counts (a
-// persistent kernel sums them over its items first): each wavefront reduces its lanes
-// (cross-lane), then one barrier, and the block's first work-item adds the wavefronts' partials
-// to the global counters — one barrier where the tree over the block's work-items takes one per
-// level. Blocks of N work-items, a multiple of 64; called by every work-item.
-template <int N>
-__device__ void add_block_counts(ne_counters* c, unsigned iters, unsigned solved, unsigned nonconv, unsigned nan,
-                                 unsigned maxit) {
-    constexpr int NW = N / 64;
-    __shared__ unsigned s_part[5][NW];
-    for (int d = 32; d >= 1; d >>= 1) {
-        iters += (unsigned)__shfl_xor((int)iters, d, 64);
-        solved += (unsigned)__shfl_xor((int)solved, d, 64);
-        nonconv += (unsigned)__shfl_xor((int)nonconv, d, 64);
-        nan += (unsigned)__shfl_xor((int)nan, d, 64);
-        const unsigned o = (unsigned)__shfl_xor((int)maxit, d, 64);
-        maxit = o > maxit ? o : maxit;
-    }
-    const int t = threadIdx.x + threadIdx.y * blockDim.x;
-    const int w = t >> 6;
-    if ((t & 63) == 0) {
-        s_part[0][w] = iters;
-        s_part[1][w] = solved;
-        s_part[2][w] = nonconv;
-        s_part[3][w] = nan;
-        s_part[4][w] = maxit;
-    }
-    __syncthreads();
-    if (t != 0 || c == nullptr) return;
-    unsigned long long tot = 0;
-    unsigned n = 0, nc = 0, nn = 0, m = 0;
-    const int nw = ((int)(blockDim.x * blockDim.y) + 63) / 64;
-    for (int k = 0; k < nw; k++) {
-        tot += s_part[0][k];
-        n += s_part[1][k];
-        nc += s_part[2][k];
-        nn += s_part[3][k];
-        m = s_part[4][k] > m ? s_part[4][k] : m;
-    }
+// Adds a wavefront's counts (per work-item; a persistent kernel sums them over its items first).
+// Called by every work-item of the block. The sums are taken bit by bit from votes, on the scalar unit.
+__device__ __forceinline__ unsigned wave_sum(unsigned x) {
+    unsigned sum = 0;
+    for (int b = 0; b < 32 && __any(x >> b); b++) sum += (unsigned)__popcll(__ballot((x >> b) & 1u)) << b;
+    return sum;
+}
+__device__ __forceinline__ unsigned wave_max(unsigned x) {
+    int b = 0;
+    while (b < 32 && __any(x >> b)) b++;
+    unsigned m = 0;
+    while (--b >= 0)
+        if (__any((x >> b) == (m >> b | 1u))) m |= 1u << b;
+    return m;
+}
+__device__ void add_wave_counts(ne_counters* c, unsigned iters, unsigned solved, unsigned nonconv, unsigned nan,
+                                unsigned maxit) {
+    if (c == nullptr) return;
+    const unsigned n = wave_sum(solved);
     if (n == 0) return;
-    atomicAdd((unsigned long long*)&c->total_iterations, tot);
+    const unsigned tot = wave_sum(iters), nc = wave_sum(nonconv), nn = wave_sum(nan), m = wave_max(maxit);
+    if (((threadIdx.x + threadIdx.y * blockDim.x) & 63) != 0) return;
+    c = counter_stripe(c);
+    atomicAdd((unsigned long long*)&c->total_iterations, (unsigned long long)tot);
     atomicAdd(&c->solved_columns, n);
     if (nc) atomicAdd(&c->nonconverged_columns, nc);
     if (nn) atomicAdd(&c->nan_columns, nn);
     atomicMax(&c->max_iterations, m);
 }
 
-// add_block_counts for a kernel with one column per work-item.
-template <int N>
-__device__ void accumulate_counters_once(ne_counters* c, bool solved, int it, bool nonconv, bool nan) {
-    add_block_counts<N>(c, solved ? (unsigned)it : 0u, solved ? 1u : 0u, (solved && nonconv) ? 1u : 0u,
-                        (solved && nan) ? 1u : 0u, solved ? (unsigned)it : 0u);
+// add_wave_counts for a kernel with one column per work-item.
+__device__ __forceinline__ void count_column(ne_counters* c, bool solved, int it, bool nonconv, bool nan) {
+    add_wave_counts(c, solved ? (unsigned)it : 0u, solved ? 1u : 0u, (solved && nonconv) ? 1u : 0u,
+                    (solved && nan) ? 1u : 0u, solved ? (unsigned)it : 0u);
 }
 
 __device__ __forceinline__ void store_fluxes(const FluxOut& o, int i, int j, const ColumnFluxes& r) {
@@ -174,6 +135,45 @@ __device__ __forceinline__ void store_fluxes(const FluxOut& o, int i, int j, con
 
 __device__ __forceinline__ bool finite3(double a, double b, double c) {
     return isfinite(a) && isfinite(b) && isfinite(c);
+}
+
+// The block's copy of the stability-function table its flux path uses (none for the general path),
+// FP32 for the mixed form's FP32 iteration; load_table is called by every work-item of the block.
+template <typename Real, int PATH>
+using FluxTable =
+    std::conditional_t<PATH == 0, NoTable,
+                       PsiTable<std::conditional_t<NE_MIXED_PREITERATION && sizeof(Real) == 4, float, double>>>;
+
+// Every load of a work-item's share is issued before the first is waited for (blocks of at least
+// MIN work-items; larger ones leave the last rounds empty).
+template <int MIN, typename T, int N>
+__device__ __forceinline__ void copy_to_lds(T (&to)[N], const T* from) {
+    const int t = threadIdx.x + threadIdx.y * blockDim.x, threads = blockDim.x * blockDim.y;
+    constexpr int ROUNDS = (N + MIN - 1) / MIN;
+    T part[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const int k = t + r * threads;
+        part[r] = from[k < N ? k : 0];
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const int k = t + r * threads;
+        if (k < N) to[k] = part[r];
+    }
+}
+template <int MIN>
+__device__ __forceinline__ void load_table(NoTable&) {}
+template <int MIN>
+__device__ __forceinline__ void load_table(PsiTable<double>& s) {
+    copy_to_lds<MIN>(s.c, reinterpret_cast<const double2*>(psi_table_f64));
+    copy_to_lds<MIN>(s.log, reinterpret_cast<const double2*>(log_table_f64));
+    __syncthreads();
+}
+template <int MIN>
+__device__ __forceinline__ void load_table(PsiTable<float>& s) {
+    copy_to_lds<MIN>(s.c, reinterpret_cast<const float4*>(psi_table_f32));
+    __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -332,16 +332,18 @@ __device__ __forceinline__ void ocean_surface(const GridDev& g, const View3<cons
     vo = ((double)v(i, j, kN) + (double)v(i, jp, kN)) / 2.0;
 }
 
-template <bool Fast, bool Consts>
+template <int PATH>
 __global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3<const double> va,
                                            View3<const double> Ta, View3<const double> pa, View3<const double> qa,
                                            View3<const double> T, View3<const double> S, View3<const double> u,
                                            View3<const double> v, View3<const double> sw,
                                            View3<const double> lw, FluxOut out, ne_counters* counters) {
+    __shared__ FluxTable<double, PATH> tab;
+    load_table<BX * BY>(tab);
     int i = blockIdx.x * BX + threadIdx.x;
     int j = blockIdx.y * BY + threadIdx.y;
-    if (out.iters.p) {   // columns in the order K1 takes them (previous iteration count, stability)
+    if (out.iters.p && PATH == 0) {   // columns in the order K1 takes them (previous iteration count, stability)
         const bool own = i < g.Nx && j < g.Ny;
         const int key = own ? solve_order_key(out, i, j) : SORT_BINS - 1;
         const int c = sorted_block_column(key, threadIdx.x + threadIdx.y * BX);
@@ -356,16 +358,16 @@ flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3
         ocean_surface<double>(g, T, S, u, v, i, j, To, So, uo, vo);
         inactive = !g.active(i, j, g.Nz - 1);
         double SW = 0.0, LW = 0.0;
-        if (!Fast && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
+        if (PATH == 0 && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
             SW = sw.at2(i, j);
             LW = lw.at2(i, j);
         }
-        r = flux_column<Fast, false, Consts>(p, ua.at2(i, j), va.at2(i, j), Ta.at2(i, j), pa.at2(i, j), qa.at2(i, j), To, uo, vo,
+        r = flux_column<PATH, false, false>(tab, p, ua.at2(i, j), va.at2(i, j), Ta.at2(i, j), pa.at2(i, j), qa.at2(i, j), To, uo, vo,
                               inactive, SW, LW);
         store_fluxes(out, i, j, r);
     }
     bool solved = in && !inactive;
-    accumulate_counters_once<BX * BY>(counters, solved, solved ? r.iterations : 0, solved && !r.converged,
+    count_column(counters, solved, solved ? r.iterations : 0, solved && !r.converged,
                                       solved && !finite3(r.us, r.ts, r.qs));
 }
 
@@ -374,12 +376,14 @@ flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3
 // the wrapped interior column (the values the reference's filled halo holds), and a ring node
 // beyond a bounded edge is inactive (zero interface state). The solve runs as in the interior
 // (same instance of the column solve); the ring is not counted in the solver counters.
-template <bool Fast, bool Consts>
+template <int PATH>
 __global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 flux_solve_ring_kernel(GridDev g, ne_params p, View3<const double> ua, View3<const double> va,
                        View3<const double> Ta, View3<const double> pa, View3<const double> qa,
                        View3<const double> T, View3<const double> S, View3<const double> u,
                        View3<const double> v, View3<const double> sw, View3<const double> lw, FluxOut out) {
+    __shared__ FluxTable<double, PATH> tab;
+    load_table<BX * BY>(tab);
     int i, j;
     if (!ring_position(g, (int)(blockIdx.x * blockDim.x + threadIdx.x), i, j)) return;
     double To = 0.0, So = 0.0, uo = 0.0, vo = 0.0;
@@ -390,11 +394,11 @@ flux_solve_ring_kernel(GridDev g, ne_params p, View3<const double> ua, View3<con
         inactive = !g.active(wi, wj, g.Nz - 1);
     }
     double SW = 0.0, LW = 0.0;
-    if (!Fast && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
+    if (PATH == 0 && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
         SW = sw.at2(i, j);
         LW = lw.at2(i, j);
     }
-    ColumnFluxes r = flux_column<Fast, false, Consts>(p, ua.at2(i, j), va.at2(i, j), Ta.at2(i, j), pa.at2(i, j),
+    ColumnFluxes r = flux_column<PATH, false, false>(tab, p, ua.at2(i, j), va.at2(i, j), Ta.at2(i, j), pa.at2(i, j),
                                                       qa.at2(i, j), To, uo, vo, inactive, SW, LW);
     store_fluxes(out, i, j, r);
 }
@@ -402,8 +406,8 @@ flux_solve_ring_kernel(GridDev g, ne_params p, View3<const double> ua, View3<con
 // One column of K1: interpolate the atmosphere at the column, solve, store the fluxes.
 // The skin-temperature balance also reads the downwelling radiation, interpolated here
 // exactly as K2 interpolates it.
-template <typename Real, bool Fast, bool Consts, bool Defer = false>
-__device__ __forceinline__ ColumnFluxes surface_solve_column(const GridDev& g, const ne_params& p,
+template <typename Real, int PATH, bool Defer, typename Tab>
+__device__ __forceinline__ ColumnFluxes surface_solve_column(const Tab& tab, const GridDev& g, const ne_params& p,
                                                              const AtmosDev<Real>& a, const double* __restrict__ fi,
                                                              const double* __restrict__ fj, const RadDev<Real>& rd,
                                                              const double* __restrict__ rfi,
@@ -422,15 +426,15 @@ __device__ __forceinline__ ColumnFluxes surface_solve_column(const GridDev& g, c
     ocean_surface<Real>(g, T, S, u, v, i, j, To, So, uo, vo);
     inactive = !g.active(i, j, g.Nz - 1);
     double SW = 0.0, LW = 0.0;
-    if (!Fast && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
+    if (PATH == 0 && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
         Neighbours rx = neighbours(rfi[i], rd.Nx, rd.tx);
         Neighbours ry = neighbours(rfj[j], rd.Ny, rd.ty);
         SW = interp_field(rd.sw, rx, ry, rd.time);
         LW = interp_field(rd.lw, rx, ry, rd.time);
     }
     // FP32 storage (the mixed form) also takes the FP32 pre-iteration of the fixed point
-    ColumnFluxes r = flux_column<Fast, NE_MIXED_PREITERATION && sizeof(Real) == 4, Consts, Defer>(
-        p, ua, va, Ta, pa, qa, To, uo, vo, inactive, SW, LW);
+    ColumnFluxes r = flux_column<PATH, NE_MIXED_PREITERATION && sizeof(Real) == 4, Defer>(
+        tab, p, ua, va, Ta, pa, qa, To, uo, vo, inactive, SW, LW);
     if (!Defer || !r.deferred) store_fluxes(out, i, j, r);
     return r;
 }
@@ -639,23 +643,25 @@ __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const 
 // Defer (FP32 storage with parameters that take the FP32 iteration): a column whose FP32
 // iteration does not finish it is appended to `deferred` (count, then flattened columns) and left
 // to surface_deferred_kernel.
-template <typename Real, bool Fast, bool Consts, bool Defer = false, int KBY = BY>
+template <typename Real, int PATH, bool Defer = false, int KBY = BY>
 __global__ void __launch_bounds__(BX* KBY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __restrict__ fi,
                       const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
                       const double* __restrict__ rfj, View3<Real> T, View3<const Real> S, View3<const Real> u,
                       View3<const Real> v, FluxOut out, NetOut n, RadOut ro, View3<double> frazil, double dt_frazil,
                       uint8_t* __restrict__ freeze_flags, ne_counters* counters, int* deferred) {
+    __shared__ FluxTable<Real, PATH> tab;
+    load_table<BX * KBY>(tab);
     int i = blockIdx.x * BX + threadIdx.x;
     int j = blockIdx.y * KBY + threadIdx.y;
-    if (out.iters.p && !Defer) {
-        // (Not for the mixed form's FP32 iteration, whose counts vary less: without the sort and
-        // its barriers its K1 took 124 → 117 µs at 1440×560×10.)
+    if (out.iters.p && PATH == 0) {
         // Columns of the block in order of the iteration count the previous solve took, the
         // stable ones last (solve_order_key): the fixed point runs until the slowest column of a
         // wavefront converges, so wavefronts of columns with like counts leave fewer lanes idle,
         // and a wavefront without stable columns skips that branch. Each column's result does
-        // not depend on the lane that computes it.
+        // not depend on the lane that computes it. Only for the general path: with the table, whose
+        // iterations are short and the same for stable and unstable columns, the sort's barriers and
+        // its gathered loads cost what it saves (FP64 1440×560×10: 174 µs with it, 173 without).
         const int t = threadIdx.x + threadIdx.y * BX;
         const bool own = i < g.Nx && j < g.Ny;
         const int key = own ? solve_order_key(out, i, j) : SORT_BINS - 1;
@@ -668,7 +674,7 @@ surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __
     r.deferred = false;
     bool inactive = true;
     if (in) {
-        r = surface_solve_column<Real, Fast, Consts, Defer>(g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i,
+        r = surface_solve_column<Real, PATH, Defer>(tab, g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i,
                                                             j, inactive);
         if (Defer && r.deferred)
             deferred[1 + atomicAdd(&deferred[0], 1)] = i + j * g.Nx;
@@ -677,14 +683,14 @@ surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __
                                                  freeze_flags, r.Qt, r.Qv, r.Jv, r.Ts_C, i, j);
     }
     bool solved = in && !inactive && !(Defer && r.deferred);
-    accumulate_counters_once<BX * KBY>(counters, solved, solved ? r.iterations : 0, solved && !r.converged,
+    count_column(counters, solved, solved ? r.iterations : 0, solved && !r.converged,
                         solved && !finite3(r.us, r.ts, r.qs));
 }
 
 // The columns surface_update_kernel deferred, finished as the kernel without deferral finishes
 // them (the FP32 iteration again, then the FP64 one): a grid-stride loop over the list, which is
 // empty in most steps. surface_tau_kernel, which runs after it, clears the count.
-template <typename Real, bool Fast, bool Consts>
+template <typename Real, int PATH>
 __global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 surface_deferred_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __restrict__ fi,
                         const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
@@ -693,7 +699,10 @@ surface_deferred_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* 
                         double dt_frazil, uint8_t* __restrict__ freeze_flags, ne_counters* counters,
                         const int* __restrict__ deferred) {
     const int count = deferred[0];   // the same for every work-item: nothing writes it meanwhile
-    // rounds of one column per work-item, uniform over the block (the counters synchronise it)
+    if (count == 0) return;
+    __shared__ FluxTable<Real, PATH> tab;
+    load_table<BX * BY>(tab);
+    // rounds of one column per work-item
     for (int base = blockIdx.x * BX * BY; base < count; base += gridDim.x * BX * BY) {
         const int q = base + (int)(threadIdx.x + threadIdx.y * BX);
         ColumnFluxes r;
@@ -701,13 +710,13 @@ surface_deferred_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* 
         if (q < count) {
             const int col = deferred[1 + q];
             const int i = col % g.Nx, j = col / g.Nx;
-            r = surface_solve_column<Real, Fast, Consts>(g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i, j,
+            r = surface_solve_column<Real, PATH, false>(tab, g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i, j,
                                                          inactive);
             surface_finalize_column<Real, false>(g, p, a, fi, fj, rd, rfi, rfj, T, S, out, n, ro, frazil,
                                                  dt_frazil, freeze_flags, r.Qt, r.Qv, r.Jv, r.Ts_C, i, j);
         }
         const bool solved = q < count && !inactive;
-        accumulate_counters(counters, solved, solved ? r.iterations : 0, solved && !r.converged,
+        count_column(counters, solved, solved ? r.iterations : 0, solved && !r.converged,
                             solved && !finite3(r.us, r.ts, r.qs));
     }
 }
@@ -734,10 +743,12 @@ __global__ void __launch_bounds__(BX* BY) surface_tau_kernel(GridDev g, ne_param
 // FUSED (the step): each column then goes on as in the single model's K1 (freeze clamp of the
 // flagged columns, net fluxes other than τ, radiation); without it (the autotuner's timing
 // runs) the kernel only solves, leaving the state as it is.
-template <typename Real, bool Fast, bool Consts, bool FUSED>
+template <typename Real, int PATH, bool FUSED>
 __global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem* __restrict__ work, int nwork,
                            double dt_frazil, ne_counters* counters) {
+    __shared__ FluxTable<Real, PATH> tab;
+    load_table<64>(tab);
     // this work-item's counts over its items, added to the counters once at the end
     unsigned n_it = 0u, n_solved = 0u, n_nc = 0u, n_nan = 0u, n_max = 0u;
     for (int wi = blockIdx.x; wi < nwork; wi += gridDim.x) {
@@ -745,9 +756,8 @@ batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkIt
         const BatchRec<Real>& rc = recs[it.member];
         const GridDev g = rc.g;
         int col = it.index + (int)threadIdx.x;
-        if (rc.f.iters.p && blockDim.x > 64 && !(sizeof(Real) == 4 && Fast)) {
-            // the item's columns in the single model's order (previous iteration count, stability;
-            // the mixed form's FP32 iteration, as there, takes them unsorted)
+        if (rc.f.iters.p && blockDim.x > 64 && PATH == 0) {
+            // the item's columns in the single model's order (previous iteration count, stability)
             const int key = col < g.Nx * g.Ny ? solve_order_key(rc.f, col % g.Nx, col / g.Nx) : SORT_BINS - 1;
             col = it.index + sorted_block_column(key, (int)threadIdx.x);
         }
@@ -757,7 +767,7 @@ batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkIt
         bool inactive = true;
         if (in)
         {
-            r = surface_solve_column<Real, Fast, Consts>(g, rc.p, rc.a, rc.afi, rc.afj, rc.r, rc.rfi, rc.rfj, cview(rc.T),
+            r = surface_solve_column<Real, PATH, false>(tab, g, rc.p, rc.a, rc.afi, rc.afj, rc.r, rc.rfi, rc.rfj, cview(rc.T),
                                                  cview(rc.S), rc.u, rc.v, rc.f, i, j, inactive);
             if (FUSED)
                 surface_finalize_column<Real, false>(g, rc.p, rc.a, rc.afi, rc.afj, rc.r, rc.rfi, rc.rfj, rc.T,
@@ -772,7 +782,7 @@ batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkIt
             n_max = (unsigned)r.iterations > n_max ? (unsigned)r.iterations : n_max;
         }
     }
-    add_block_counts<BX * BY>(counters, n_it, n_solved, n_nc, n_nan, n_max);
+    add_wave_counts(counters, n_it, n_solved, n_nc, n_nan, n_max);
 }
 
 // Ensemble form of K2 over the same work list as the ensemble K1: τ of every column.
@@ -934,15 +944,19 @@ hipError_t launch_flux_solve_exchange(const GridDev& g, const ne_params& p, cons
     View3<const double> sw = view<const double>(a.downwelling_shortwave);
     View3<const double> lw = view<const double>(a.downwelling_longwave);
     const int path = flux_path(p);
-    auto kernel = path == 2 ? flux_solve_exchange_kernel<true, true>
-                : path == 1 ? flux_solve_exchange_kernel<true, false> : flux_solve_exchange_kernel<false, false>;
+    auto kernel = path == 2   ? flux_solve_exchange_kernel<2>
+                  : path == 3 ? flux_solve_exchange_kernel<3>
+                  : path == 1 ? flux_solve_exchange_kernel<1>
+                              : flux_solve_exchange_kernel<0>;
     hipLaunchKernelGGL(kernel, grid2d(g.Nx, g.Ny), dim3(BX, BY), 0, s, g, p, view<const double>(a.u),
                        view<const double>(a.v), view<const double>(a.T), view<const double>(a.p),
                        view<const double>(a.q), view<const double>(o.T), view<const double>(o.S),
                        view<const double>(o.u), view<const double>(o.v), sw, lw, out, c);
     if (g.ring) {
-        auto ring = path == 2 ? flux_solve_ring_kernel<true, true>
-                  : path == 1 ? flux_solve_ring_kernel<true, false> : flux_solve_ring_kernel<false, false>;
+        auto ring = path == 2   ? flux_solve_ring_kernel<2>
+                    : path == 3 ? flux_solve_ring_kernel<3>
+                    : path == 1 ? flux_solve_ring_kernel<1>
+                                : flux_solve_ring_kernel<0>;
         hipLaunchKernelGGL(ring, dim3((ring_size(g) + BX * BY - 1) / (BX * BY)), dim3(BX * BY), 0, s, g, p,
                            view<const double>(a.u), view<const double>(a.v), view<const double>(a.T),
                            view<const double>(a.p), view<const double>(a.q), view<const double>(o.T),
@@ -994,9 +1008,12 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
         // the FP32 iteration alone at 6 wavefronts per SIMD in blocks of 8 rows, then the deferred
         // columns
         constexpr int KBY = NE_FLUX_MIXED_ROWS;
-        auto k1 = path == 2 ? surface_update_kernel<Real, true, true, true, KBY>
-                            : surface_update_kernel<Real, true, false, true, KBY>;
-        auto k2 = path == 2 ? surface_deferred_kernel<Real, true, true> : surface_deferred_kernel<Real, true, false>;
+        auto k1 = path == 2   ? surface_update_kernel<Real, 2, true, KBY>
+                  : path == 3 ? surface_update_kernel<Real, 3, true, KBY>
+                              : surface_update_kernel<Real, 1, true, KBY>;
+        auto k2 = path == 2   ? surface_deferred_kernel<Real, 2>
+                  : path == 3 ? surface_deferred_kernel<Real, 3>
+                              : surface_deferred_kernel<Real, 1>;
         hipLaunchKernelGGL(k1, dim3((g.Nx + BX - 1) / BX, (g.Ny + KBY - 1) / KBY), dim3(BX, KBY), 0, s, g, p, a, fi, fj,
                            r, rfi, rfj, T, S, u, v, out, n, ro, frazil, dt_frazil, freeze_flags, c, deferred);
         const unsigned blocks = std::min<unsigned>(grid.x * grid.y, 256u);
@@ -1004,8 +1021,10 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
                            frazil, dt_frazil, freeze_flags, c, deferred);
         return hipGetLastError();
     }
-    auto kernel = path == 2 ? surface_update_kernel<Real, true, true>
-                : path == 1 ? surface_update_kernel<Real, true, false> : surface_update_kernel<Real, false, false>;
+    auto kernel = path == 2   ? surface_update_kernel<Real, 2>
+                  : path == 3 ? surface_update_kernel<Real, 3>
+                  : path == 1 ? surface_update_kernel<Real, 1>
+                              : surface_update_kernel<Real, 0>;
     hipLaunchKernelGGL(kernel, grid, dim3(BX, BY), 0, s, g, p, a, fi, fj, r, rfi, rfj, T, S, u, v, out, n, ro, frazil,
                        dt_frazil, freeze_flags, c, (int*)nullptr);
     return hipGetLastError();
@@ -1037,8 +1056,10 @@ hipError_t launch_batch_surface_solve(const BatchRec<Real>* recs, const WorkItem
     if (block <= 0 || block > BX * BY || (block & (block - 1)) != 0 || blocks <= 0) return hipErrorInvalidValue;
     auto pick = [&](auto fused_tag) {
         constexpr bool F = decltype(fused_tag)::value;
-        return path == 2 ? batch_surface_solve_kernel<Real, true, true, F>
-             : path == 1 ? batch_surface_solve_kernel<Real, true, false, F> : batch_surface_solve_kernel<Real, false, false, F>;
+        return path == 2   ? batch_surface_solve_kernel<Real, 2, F>
+               : path == 3 ? batch_surface_solve_kernel<Real, 3, F>
+               : path == 1 ? batch_surface_solve_kernel<Real, 1, F>
+                           : batch_surface_solve_kernel<Real, 0, F>;
     };
     auto kernel = fused ? pick(std::true_type{}) : pick(std::false_type{});
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(block), 0, s, recs, work, nwork, dt_frazil, c);
