@@ -185,7 +185,7 @@ BatchRec<Real> member_record(const ne_model* m, const double* atimes_dev, const 
     return r;
 }
 
-// Host-side layout of the arena: records | times | 2×3 stage lists | 3 surface lists | 4×3 solve lists.
+// Host-side layout of the arena: records | times | 2×3 stage lists | 3 surface lists | 5×3 solve lists.
 struct Layout {
     size_t recs = 0, times = 0, stage[2][3] = {{0, 0, 0}, {0, 0, 0}}, surface[3] = {0, 0, 0},
            solve[FLUX_PATHS][3] = {};

@@ -141,7 +141,7 @@ __device__ __forceinline__ bool finite3(double a, double b, double c) {
 // FP32 for the mixed form's FP32 iteration; load_table is called by every work-item of the block.
 template <typename Real, int PATH>
 using FluxTable =
-    std::conditional_t<PATH == 0, NoTable,
+    std::conditional_t<PATH == 0 || PATH == 4, NoTable,
                        PsiTable<std::conditional_t<NE_MIXED_PREITERATION && sizeof(Real) == 4, float, double>>>;
 
 // Every load of a work-item's share is issued before the first is waited for (blocks of at least
@@ -343,7 +343,7 @@ flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3
     load_table<BX * BY>(tab);
     int i = blockIdx.x * BX + threadIdx.x;
     int j = blockIdx.y * BY + threadIdx.y;
-    if (out.iters.p && PATH == 0) {   // columns in the order K1 takes them (previous iteration count, stability)
+    if (out.iters.p && (PATH == 0 || PATH == 4)) {   // columns in the order K1 takes them (previous iteration count, stability)
         const bool own = i < g.Nx && j < g.Ny;
         const int key = own ? solve_order_key(out, i, j) : SORT_BINS - 1;
         const int c = sorted_block_column(key, threadIdx.x + threadIdx.y * BX);
@@ -654,7 +654,7 @@ surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __
     load_table<BX * KBY>(tab);
     int i = blockIdx.x * BX + threadIdx.x;
     int j = blockIdx.y * KBY + threadIdx.y;
-    if (out.iters.p && PATH == 0) {
+    if (out.iters.p && (PATH == 0 || PATH == 4)) {
         // Columns of the block in order of the iteration count the previous solve took, the
         // stable ones last (solve_order_key): the fixed point runs until the slowest column of a
         // wavefront converges, so wavefronts of columns with like counts leave fewer lanes idle,
@@ -756,7 +756,7 @@ batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkIt
         const BatchRec<Real>& rc = recs[it.member];
         const GridDev g = rc.g;
         int col = it.index + (int)threadIdx.x;
-        if (rc.f.iters.p && blockDim.x > 64 && PATH == 0) {
+        if (rc.f.iters.p && blockDim.x > 64 && (PATH == 0 || PATH == 4)) {
             // the item's columns in the single model's order (previous iteration count, stability)
             const int key = col < g.Nx * g.Ny ? solve_order_key(rc.f, col % g.Nx, col / g.Nx) : SORT_BINS - 1;
             col = it.index + sorted_block_column(key, (int)threadIdx.x);
@@ -946,6 +946,7 @@ hipError_t launch_flux_solve_exchange(const GridDev& g, const ne_params& p, cons
     const int path = flux_path(p);
     auto kernel = path == 2   ? flux_solve_exchange_kernel<2>
                   : path == 3 ? flux_solve_exchange_kernel<3>
+                  : path == 4 ? flux_solve_exchange_kernel<4>
                   : path == 1 ? flux_solve_exchange_kernel<1>
                               : flux_solve_exchange_kernel<0>;
     hipLaunchKernelGGL(kernel, grid2d(g.Nx, g.Ny), dim3(BX, BY), 0, s, g, p, view<const double>(a.u),
@@ -955,6 +956,7 @@ hipError_t launch_flux_solve_exchange(const GridDev& g, const ne_params& p, cons
     if (g.ring) {
         auto ring = path == 2   ? flux_solve_ring_kernel<2>
                     : path == 3 ? flux_solve_ring_kernel<3>
+                    : path == 4 ? flux_solve_ring_kernel<4>
                     : path == 1 ? flux_solve_ring_kernel<1>
                                 : flux_solve_ring_kernel<0>;
         hipLaunchKernelGGL(ring, dim3((ring_size(g) + BX * BY - 1) / (BX * BY)), dim3(BX * BY), 0, s, g, p,
@@ -1004,7 +1006,8 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
                                  hipStream_t s) {
     const int path = flux_path(p);
     const dim3 grid = grid2d(g.Nx, g.Ny);
-    if (sizeof(Real) == 4 && path >= 1 && deferred && mixed_iteration_applies(p)) {
+    if constexpr (sizeof(Real) == 4)
+    if (path >= 1 && path <= 3 && deferred && mixed_iteration_applies(p)) {
         // the FP32 iteration alone at 6 wavefronts per SIMD in blocks of 8 rows, then the deferred
         // columns
         constexpr int KBY = NE_FLUX_MIXED_ROWS;
@@ -1023,6 +1026,7 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
     }
     auto kernel = path == 2   ? surface_update_kernel<Real, 2>
                   : path == 3 ? surface_update_kernel<Real, 3>
+                  : path == 4 ? surface_update_kernel<Real, 4>
                   : path == 1 ? surface_update_kernel<Real, 1>
                               : surface_update_kernel<Real, 0>;
     hipLaunchKernelGGL(kernel, grid, dim3(BX, BY), 0, s, g, p, a, fi, fj, r, rfi, rfj, T, S, u, v, out, n, ro, frazil,
@@ -1058,6 +1062,7 @@ hipError_t launch_batch_surface_solve(const BatchRec<Real>* recs, const WorkItem
         constexpr bool F = decltype(fused_tag)::value;
         return path == 2   ? batch_surface_solve_kernel<Real, 2, F>
                : path == 3 ? batch_surface_solve_kernel<Real, 3, F>
+               : path == 4 ? batch_surface_solve_kernel<Real, 4, F>
                : path == 1 ? batch_surface_solve_kernel<Real, 1, F>
                            : batch_surface_solve_kernel<Real, 0, F>;
     };
