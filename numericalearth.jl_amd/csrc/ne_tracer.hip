@@ -102,15 +102,12 @@ inline int grid_blocks(const GridDev& g, int levels) {
 // three are packed in 10-bit fields of one register (grids have at most NE_MAX_LEVELS =
 // 1023 levels, so 1023 — "never" — exceeds every level).
 constexpr uint32_t NEVER_LEVEL = 1023u;
-__device__ __forceinline__ int order_at(int k, uint32_t P) {
-    return (k >= (int)(P & 1023u) ? 1 : 0) + (k >= (int)((P >> 10) & 1023u) ? 1 : 0) + (k >= (int)(P >> 20) ? 1 : 0);
-}
-
-// Face order at the top of level k of a column with active levels kmin … Nz-1.
-__device__ __forceinline__ int z_order(int k, int kmin, int Nz) {
-    return (k >= kmin && k <= Nz - 2 ? 1 : 0) + (k >= kmin + 1 && k <= Nz - 3 ? 1 : 0) +
-           (k >= kmin + 2 && k <= Nz - 4 ? 1 : 0);
-}
+__device__ __forceinline__ bool open_at(int k, uint32_t P) { return (uint32_t)k >= (P & 1023u); }
+__device__ __forceinline__ bool three_at(int k, uint32_t P) { return (uint32_t)k >= ((P >> 10) & 1023u); }
+__device__ __forceinline__ bool five_at(int k, uint32_t P) { return (uint32_t)k >= (P >> 20); }
+// Order (0 … 3) of the face at the top of level k of a column with active levels kmin … Nz-1: one more
+// than the levels below k, at most what the levels above allow (Nz − 1 − k, uniform).
+__device__ __forceinline__ int z_order(int k, int kmin, int Nz) { return max(min(k - kmin + 1, min(Nz - 1 - k, 3)), 0); }
 
 __device__ __forceinline__ uint32_t thresholds(const int* km, int stride) {
     const int K1 = max(km[2 * stride], km[3 * stride]);
@@ -382,8 +379,8 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
         const R bT = ldb(Tin, coff + kz), bS = ldb(Sin, coff + kz);
         const int order = z_order(kstart - 1, mykmin, Nz);
         if (cell && order > 0) {
-            FzT = (R)Azc * wb * face_value(bT, zT[0], zT[1], zT[2], zT[3], zT[4], order, wb);
-            FzS = (R)Azc * wb * face_value(bS, zS[0], zS[1], zS[2], zS[3], zS[4], order, wb);
+            FzT = (R)Azc * wb * face_value(bT, zT[0], zT[1], zT[2], zT[3], zT[4], order >= 2, order == 3, wb);
+            FzS = (R)Azc * wb * face_value(bS, zS[0], zS[1], zS[2], zS[3], zS[4], order >= 2, order == 3, wb);
         }
     }
     for (int k = kstart; k < k1; k++) {
@@ -414,16 +411,14 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
         // its 7-wavefront register budget.
         constexpr int FACE_UNROLL = sizeof(R) == 8 ? 2 : 1;
         {
-            const int order = order_at(k, Xk);
+            const bool open = open_at(k, Xk), three = three_at(k, Xk), five = five_at(k, Xk);
             const R A = (R)Axf * dzk;
             const int base = (row + 3) * PXW + lane;
 #pragma unroll FACE_UNROLL
             for (int tr = 0; tr < 2; tr++) {
                 const R* t = (tr ? sh.cS : sh.cT) + base;
                 R f = (R)0;
-                if (order > 0) {
-                    f = A * nu * face_value(t[0], t[1], t[2], t[3], t[4], t[5], order, nu);
-                }
+                if (open) f = A * nu * face_value(t[0], t[1], t[2], t[3], t[4], t[5], three, five, nu);
                 (tr ? sh.fxS : sh.fxT)[row * TW + lane] = f;
             }
         }
@@ -436,13 +431,14 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
                 const int tr = (TR >= 2 && side) ? row : (pass & 1);
                 const int r0 = side ? TR : row;           // plane row of the first stencil cell
                 const double Ay = side ? Ayn : Ays;
-                const int order = order_at(k, side ? Nk : Sk);
+                const uint32_t P = side ? Nk : Sk;
                 R f = (R)0;
-                if (order > 0) {
+                if (open_at(k, P)) {
                     const R vel = side ? nvn : nv;
                     const R A = (R)Ay * dzk;
                     const R* t = (tr ? sh.cS : sh.cT) + r0 * PXW + lane + 3;
-                    f = A * vel * face_value(t[0], t[PXW], t[2 * PXW], t[3 * PXW], t[4 * PXW], t[5 * PXW], order, vel);
+                    f = A * vel * face_value(t[0], t[PXW], t[2 * PXW], t[3 * PXW], t[4 * PXW], t[5 * PXW], three_at(k, P),
+                                             five_at(k, P), vel);
                 }
                 (tr ? sh.fyS : sh.fyT)[r0 * TC + lane] = f;
             }
@@ -452,8 +448,8 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
         const int zorder = (cell && adv) ? z_order(k, mykmin, Nz) : 0;
         R FztT = (R)0, FztS = (R)0;
         if (zorder > 0) {
-            FztT = (R)Azc * nw * face_value(zT[0], zT[1], zT[2], zT[3], zT[4], zT[5], zorder, nw);
-            FztS = (R)Azc * nw * face_value(zS[0], zS[1], zS[2], zS[3], zS[4], zS[5], zorder, nw);
+            FztT = (R)Azc * nw * face_value(zT[0], zT[1], zT[2], zT[3], zT[4], zT[5], zorder >= 2, zorder == 3, nw);
+            FztS = (R)Azc * nw * face_value(zS[0], zS[1], zS[2], zS[3], zS[4], zS[5], zorder >= 2, zorder == 3, nw);
         }
         load_w(kn);
         __syncthreads();
