@@ -79,6 +79,8 @@ struct ne_batch {
     WorkItem* solve_work[FLUX_PATHS][3] = {};   // [flux path][choice]
     int solve_nwork[FLUX_PATHS][3] = {};
 
+    bool unit = false;   // every member's fields have the unit layouts
+
     ne_batch_tuning tuning;
     int cus = 256;
     bool use_graph = false;
@@ -126,7 +128,7 @@ hipError_t enqueue_step(ne_batch* b, double dt, hipStream_t s, ne_counters* coun
         int nw = b->solve_nwork[path][si];
         e = launch_batch_surface_solve<Real>(recs, b->solve_work[path][si], nw, t.surface_block,
                                              std::min(blocks_for(t.surface_blocks, nw), std::max(nw, 1)), path,
-                                             true, dt, counters, s);
+                                             b->unit, true, dt, counters, s);
         if (e != hipSuccess) return e;
     }
     int nsu = b->surface_nwork[si];
@@ -294,6 +296,11 @@ int rebuild(ne_batch* b, hipStream_t s) {
         recs[k] = member_record<Real>(m, m->atimes.empty() ? nullptr : tdev + aoff[k],
                                       m->rtimes.empty() ? nullptr : tdev + roff[k], tile_levels);
     }
+    b->unit = true;
+    for (int k = 0; k < n; k++) {
+        const BatchRec<Real>& r = recs[k];
+        b->unit = b->unit && unit_fields<Real>(r.g, r.a, r.r, cview(r.T), cview(r.S), r.u, r.v, r.f, r.n, r.ro, r.frazil);
+    }
     if (!times.empty()) memcpy(H + L.times, times.data(), times.size() * sizeof(double));
     auto put = [&](size_t o, const std::vector<WorkItem>& w, WorkItem** view, int* count) {
         if (!w.empty()) memcpy(H + o, w.data(), w.size() * sizeof(WorkItem));
@@ -411,7 +418,7 @@ int autotune(ne_batch* b, hipStream_t s, ne_batch_tuning* out) {
                     int nw = b->solve_nwork[path][c];
                     e = launch_batch_surface_solve<Real>(recs, b->solve_work[path][c], nw, SURFACE_BLOCKS[c],
                                                          std::min(blocks_for(req, nw), std::max(nw, 1)), path,
-                                                         false, 0.0, nullptr, s);
+                                                         b->unit, false, 0.0, nullptr, s);
                 }
                 return e;
             };

@@ -64,6 +64,24 @@ __host__ inline View3<T> view(const ne_view& v) {
     return r;
 }
 
+// A column of the 2-D fields. In kernels instantiated for fields of one layout (UNIT: unit stride in
+// i, one row stride, less than 4 GiB each; unit_fields in ne_surface.hip) every field's value of the
+// column is at the same byte offset o8 from its base (half of it for 4-byte values), computed once;
+// otherwise each view's own 64-bit strides are used.
+struct Place {
+    int i, j;
+    uint32_t o8;
+};
+template <bool UNIT, typename T>
+__device__ __forceinline__ T& at(const View3<T>& v, const Place& c) {
+    if constexpr (UNIT) {
+        using Byte = std::conditional_t<std::is_const<T>::value, const char, char>;
+        return *reinterpret_cast<T*>(reinterpret_cast<Byte*>(v.p) + (sizeof(T) == 8 ? c.o8 : c.o8 >> 1));
+    } else {
+        return v.at2(c.i, c.j);
+    }
+}
+
 // Julia's min/max on floats: NaN-propagating, -0.0 < +0.0. Written as selects without early
 // returns: branches here become divergent blocks that assign a literal operand, for which the
 // compiler holds 64-bit constants in (spilled) vector registers inside the flux iteration.
@@ -1292,6 +1310,49 @@ __device__ __forceinline__ double interp_field(const View3<const Real>& d, const
     double b = w00 * (double)d(x.lo, y.lo, t.n2) + w01 * (double)d(x.lo, y.hi, t.n2) +
                w10 * (double)d(x.hi, y.lo, t.n2) + w11 * (double)d(x.hi, y.hi, t.n2);
     return (1.0 - t.tilde_n) * a + t.tilde_n * b;
+}
+
+// Where a column interpolates a source grid's fields: with UNIT (the fields share one layout, as
+// above) the four corners' byte offsets within a snapshot, the same for every field.
+template <bool UNIT>
+struct Corners {
+    Neighbours x, y;
+    uint32_t o00, o01, o10, o11;
+};
+template <bool UNIT, typename Real>
+__device__ __forceinline__ Corners<UNIT> corners(const View3<const Real>& layout, double fx, int nx, int tx, double fy,
+                                                 int ny, int ty) {
+    Corners<UNIT> c;
+    c.x = neighbours(fx, nx, tx);
+    c.y = neighbours(fy, ny, ty);
+    if constexpr (UNIT) {
+        const uint32_t sy = (uint32_t)layout.sy;
+        const uint32_t lo = (uint32_t)c.y.lo * sy, hi = (uint32_t)c.y.hi * sy;
+        c.o00 = (lo + (uint32_t)c.x.lo) * (uint32_t)sizeof(Real);
+        c.o01 = (hi + (uint32_t)c.x.lo) * (uint32_t)sizeof(Real);
+        c.o10 = (lo + (uint32_t)c.x.hi) * (uint32_t)sizeof(Real);
+        c.o11 = (hi + (uint32_t)c.x.hi) * (uint32_t)sizeof(Real);
+    }
+    return c;
+}
+// interp_field at such corners: the same operations.
+template <bool UNIT, typename Real>
+__device__ __forceinline__ double interp_at(const View3<const Real>& d, const Corners<UNIT>& c, const ne_time_interp& t) {
+    if constexpr (!UNIT) {
+        return interp_field(d, c.x, c.y, t);
+    } else {
+        if (d.p == nullptr) return 0.0;
+        const double xi = c.x.w, eta = c.y.w;
+        const double w00 = (1.0 - xi) * (1.0 - eta), w01 = (1.0 - xi) * eta, w10 = xi * (1.0 - eta), w11 = xi * eta;
+        auto value = [](const Real* base, uint32_t o) {
+            return (double)*reinterpret_cast<const Real*>(reinterpret_cast<const char*>(base) + o);
+        };
+        const Real* p1 = d.p + (int64_t)t.n1 * d.sz;
+        const Real* p2 = d.p + (int64_t)t.n2 * d.sz;
+        const double a = w00 * value(p1, c.o00) + w01 * value(p1, c.o01) + w10 * value(p1, c.o10) + w11 * value(p1, c.o11);
+        const double b = w00 * value(p2, c.o00) + w01 * value(p2, c.o01) + w10 * value(p2, c.o10) + w11 * value(p2, c.o11);
+        return (1.0 - t.tilde_n) * a + t.tilde_n * b;
+    }
 }
 
 // cpu_interpolating_time_indices (interpolate_atmospheric_state.jl:57-60): linear between

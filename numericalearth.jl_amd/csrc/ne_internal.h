@@ -157,6 +157,11 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
                                  const FluxOut& out, const NetOut& n, const RadOut& ro, View3<double> frazil,
                                  double dt_frazil, uint8_t* freeze_flags, ne_counters* c, int* deferred,
                                  hipStream_t s);
+// Whether the model's fields have the layouts that the kernels address with shared 32-bit offsets.
+template <typename Real>
+bool unit_fields(const GridDev& g, const AtmosDev<Real>& a, const RadDev<Real>& r, View3<const Real> T,
+                 View3<const Real> S, View3<const Real> u, View3<const Real> v, const FluxOut& f, const NetOut& n,
+                 const RadOut& ro, View3<double> frazil);
 // deferred (FP32 storage; nullptr: none): count + one int per column for the columns K1 leaves to
 // its second kernel; the τ kernel, which runs after both, clears the count.
 hipError_t launch_surface_tau(const GridDev& g, const ne_params& p, const FluxOut& f, const NetOut& n,
@@ -300,7 +305,7 @@ hipError_t launch_batch_stage(const BatchRec<Real>* recs, const WorkItem* work, 
                               int blocks, int stage, double beta_dt, bool two_color, hipStream_t s);
 template <typename Real>
 hipError_t launch_batch_surface_solve(const BatchRec<Real>* recs, const WorkItem* work, int nwork, int block,
-                                      int blocks, int path, bool fused, double dt_frazil, ne_counters* c,
+                                      int blocks, int path, bool unit, bool fused, double dt_frazil, ne_counters* c,
                                       hipStream_t s);
 template <typename Real>
 hipError_t launch_batch_surface_tau(const BatchRec<Real>* recs, const WorkItem* work, int nwork, int block,

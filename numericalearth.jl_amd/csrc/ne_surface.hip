@@ -120,17 +120,24 @@ __device__ __forceinline__ void count_column(ne_counters* c, bool solved, int it
                     (solved && nan) ? 1u : 0u, solved ? (unsigned)it : 0u);
 }
 
-__device__ __forceinline__ void store_fluxes(const FluxOut& o, int i, int j, const ColumnFluxes& r) {
-    o.Qv.at2(i, j) = r.Qv;
-    o.Qt.at2(i, j) = r.Qt;
-    o.Jv.at2(i, j) = r.Jv;
-    o.rtx.at2(i, j) = r.rtx;
-    o.rty.at2(i, j) = r.rty;
-    o.us.at2(i, j) = r.us;
-    o.ts.at2(i, j) = r.ts;
-    o.qs.at2(i, j) = r.qs;
-    o.Ts.at2(i, j) = r.Ts_C;
-    if (o.iters.p) o.iters.at2(i, j) = r.iterations;
+template <bool UNIT>
+__device__ __forceinline__ void store_fluxes(const FluxOut& o, const Place& c, const ColumnFluxes& r) {
+    at<UNIT>(o.Qv, c) = r.Qv;
+    at<UNIT>(o.Qt, c) = r.Qt;
+    at<UNIT>(o.Jv, c) = r.Jv;
+    at<UNIT>(o.rtx, c) = r.rtx;
+    at<UNIT>(o.rty, c) = r.rty;
+    at<UNIT>(o.us, c) = r.us;
+    at<UNIT>(o.ts, c) = r.ts;
+    at<UNIT>(o.qs, c) = r.qs;
+    at<UNIT>(o.Ts, c) = r.Ts_C;
+    if (o.iters.p) at<UNIT>(o.iters, c) = r.iterations;
+}
+
+// The column (i, j) of fields with the row stride of `layout`.
+template <bool UNIT>
+__device__ __forceinline__ Place place(const View3<double>& layout, int i, int j) {
+    return {i, j, UNIT ? ((uint32_t)i + (uint32_t)j * (uint32_t)layout.sy) * 8u : 0u};
 }
 
 __device__ __forceinline__ bool finite3(double a, double b, double c) {
@@ -319,20 +326,30 @@ __global__ void interp_radiation_ring_kernel(GridDev g, RadDev<Real> r, const do
 
 // Ocean surface values of a column: T, S at k = Nz and ℑxᶜᵃᵃ u, ℑyᵃᶜᵃ v
 // (atmosphere_ocean_fluxes.jl:62-71).
-template <typename Real>
+template <typename Real, bool UNIT>
 __device__ __forceinline__ void ocean_surface(const GridDev& g, const View3<const Real>& T, const View3<const Real>& S,
                                               const View3<const Real>& u, const View3<const Real>& v, int i, int j,
                                               double& To, double& So, double& uo, double& vo) {
     int kN = g.Nz - 1;
-    To = (double)T(i, j, kN);
-    So = (double)S(i, j, kN);
     int ip = g.tx == NE_PERIODIC ? wrap_near(i + 1, g.Nx) : i + 1;
     int jp = g.ty == NE_PERIODIC ? wrap_near(j + 1, g.Ny) : j + 1;
-    uo = ((double)u(i, j, kN) + (double)u(ip, j, kN)) / 2.0;
-    vo = ((double)v(i, j, kN) + (double)v(i, jp, kN)) / 2.0;
+    // UNIT: every view spans less than 4 GiB, so byte offsets from the top level's base fit 32 bits
+    auto top = [kN](const View3<const Real>& c, int ii, int jj) {
+        if constexpr (UNIT) {
+            const char* base = reinterpret_cast<const char*>(c.p + (int64_t)kN * c.sz);
+            return (double)*reinterpret_cast<const Real*>(
+                base + ((uint32_t)ii + (uint32_t)jj * (uint32_t)c.sy) * (uint32_t)sizeof(Real));
+        } else {
+            return (double)c(ii, jj, kN);
+        }
+    };
+    To = top(T, i, j);
+    So = top(S, i, j);
+    uo = (top(u, i, j) + top(u, ip, j)) / 2.0;
+    vo = (top(v, i, j) + top(v, i, jp)) / 2.0;
 }
 
-template <int PATH>
+template <int PATH, bool UNIT>
 __global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3<const double> va,
                                            View3<const double> Ta, View3<const double> pa, View3<const double> qa,
@@ -355,16 +372,17 @@ flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3
     bool inactive = true;
     if (in) {
         double To, So, uo, vo;
-        ocean_surface<double>(g, T, S, u, v, i, j, To, So, uo, vo);
+        const Place c = place<UNIT>(out.Qv, i, j);
+        ocean_surface<double, UNIT>(g, T, S, u, v, i, j, To, So, uo, vo);
         inactive = !g.active(i, j, g.Nz - 1);
         double SW = 0.0, LW = 0.0;
         if (PATH == 0 && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
-            SW = sw.at2(i, j);
-            LW = lw.at2(i, j);
+            SW = at<UNIT>(sw, c);
+            LW = at<UNIT>(lw, c);
         }
-        r = flux_column<PATH, false, false>(tab, p, ua.at2(i, j), va.at2(i, j), Ta.at2(i, j), pa.at2(i, j), qa.at2(i, j), To, uo, vo,
-                              inactive, SW, LW);
-        store_fluxes(out, i, j, r);
+        r = flux_column<PATH, false, false>(tab, p, at<UNIT>(ua, c), at<UNIT>(va, c), at<UNIT>(Ta, c), at<UNIT>(pa, c),
+                                            at<UNIT>(qa, c), To, uo, vo, inactive, SW, LW);
+        store_fluxes<UNIT>(out, c, r);
     }
     bool solved = in && !inactive;
     count_column(counters, solved, solved ? r.iterations : 0, solved && !r.converged,
@@ -390,7 +408,7 @@ flux_solve_ring_kernel(GridDev g, ne_params p, View3<const double> ua, View3<con
     bool inactive = true;
     if (g.column(i, j) >= 0) {
         const int wi = g.wx(i), wj = g.wy(j);
-        ocean_surface<double>(g, T, S, u, v, wi, wj, To, So, uo, vo);
+        ocean_surface<double, false>(g, T, S, u, v, wi, wj, To, So, uo, vo);
         inactive = !g.active(wi, wj, g.Nz - 1);
     }
     double SW = 0.0, LW = 0.0;
@@ -400,13 +418,13 @@ flux_solve_ring_kernel(GridDev g, ne_params p, View3<const double> ua, View3<con
     }
     ColumnFluxes r = flux_column<PATH, false, false>(tab, p, ua.at2(i, j), va.at2(i, j), Ta.at2(i, j), pa.at2(i, j),
                                                       qa.at2(i, j), To, uo, vo, inactive, SW, LW);
-    store_fluxes(out, i, j, r);
+    store_fluxes<false>(out, Place{i, j, 0u}, r);
 }
 
 // One column of K1: interpolate the atmosphere at the column, solve, store the fluxes.
 // The skin-temperature balance also reads the downwelling radiation, interpolated here
 // exactly as K2 interpolates it.
-template <typename Real, int PATH, bool Defer, typename Tab>
+template <typename Real, int PATH, bool UNIT, bool Defer, typename Tab>
 __device__ __forceinline__ ColumnFluxes surface_solve_column(const Tab& tab, const GridDev& g, const ne_params& p,
                                                              const AtmosDev<Real>& a, const double* __restrict__ fi,
                                                              const double* __restrict__ fj, const RadDev<Real>& rd,
@@ -415,27 +433,25 @@ __device__ __forceinline__ ColumnFluxes surface_solve_column(const Tab& tab, con
                                                              const View3<const Real>& T, const View3<const Real>& S,
                                                              const View3<const Real>& u, const View3<const Real>& v,
                                                              const FluxOut& out, int i, int j, bool& inactive) {
-    Neighbours x = neighbours(fi[i], a.Nx, a.tx);
-    Neighbours y = neighbours(fj[j], a.Ny, a.ty);
-    double ua = interp_field(a.u, x, y, a.time);
-    double va = interp_field(a.v, x, y, a.time);
-    double Ta = interp_field(a.T, x, y, a.time);
-    double pa = interp_field(a.p, x, y, a.time);
-    double qa = interp_field(a.q, x, y, a.time);
+    const Corners<UNIT> c = corners<UNIT>(a.T, fi[i], a.Nx, a.tx, fj[j], a.Ny, a.ty);
+    double ua = interp_at(a.u, c, a.time);
+    double va = interp_at(a.v, c, a.time);
+    double Ta = interp_at(a.T, c, a.time);
+    double pa = interp_at(a.p, c, a.time);
+    double qa = interp_at(a.q, c, a.time);
     double To, So, uo, vo;
-    ocean_surface<Real>(g, T, S, u, v, i, j, To, So, uo, vo);
+    ocean_surface<Real, UNIT>(g, T, S, u, v, i, j, To, So, uo, vo);
     inactive = !g.active(i, j, g.Nz - 1);
     double SW = 0.0, LW = 0.0;
     if (PATH == 0 && p.interface_temperature == NE_TEMPERATURE_SKIN && p.radiation) {
-        Neighbours rx = neighbours(rfi[i], rd.Nx, rd.tx);
-        Neighbours ry = neighbours(rfj[j], rd.Ny, rd.ty);
-        SW = interp_field(rd.sw, rx, ry, rd.time);
-        LW = interp_field(rd.lw, rx, ry, rd.time);
+        const Corners<UNIT> rc = corners<UNIT>(rd.sw, rfi[i], rd.Nx, rd.tx, rfj[j], rd.Ny, rd.ty);
+        SW = interp_at(rd.sw, rc, rd.time);
+        LW = interp_at(rd.lw, rc, rd.time);
     }
     // FP32 storage (the mixed form) also takes the FP32 pre-iteration of the fixed point
     ColumnFluxes r = flux_column<PATH, NE_MIXED_PREITERATION && sizeof(Real) == 4, Defer>(
         tab, p, ua, va, Ta, pa, qa, To, uo, vo, inactive, SW, LW);
-    if (!Defer || !r.deferred) store_fluxes(out, i, j, r);
+    if (!Defer || !r.deferred) store_fluxes<UNIT>(out, place<UNIT>(out.Qv, i, j), r);
     return r;
 }
 
@@ -526,10 +542,11 @@ __device__ __forceinline__ double radiation_column(const ne_params& p, double Ts
     return SQ * rinv * cinv;
 }
 
-__device__ __forceinline__ void store_penetrating_shortwave(const ne_params& p, const NetOut& n, int i, int j,
+template <bool UNIT>
+__device__ __forceinline__ void store_penetrating_shortwave(const ne_params& p, const NetOut& n, const Place& c,
                                                             double Itsw) {
     if (p.radiative_forcing == NE_RADIATIVE_FORCING_TWO_COLOR)
-        n.J_sw.at2(i, j) = -Itsw / (p.ocean_reference_density * p.ocean_heat_capacity);
+        at<UNIT>(n.J_sw, c) = -Itsw / (p.ocean_reference_density * p.ocean_heat_capacity);
 }
 
 // Momentum fluxes of the west / south neighbours (zero state outside the domain).
@@ -570,21 +587,20 @@ __global__ void radiation_kernel(GridDev g, ne_params p, View3<const double> sw,
     double JTrad = radiation_column(p, Ts.at2(i, j), sw.at2(i, j), lw.at2(i, j), Iup, Ila, Itsw);
     bool inactive = !g.active(i, j, g.Nz - 1);
     n.J_T.at2(i, j) = n.J_T.at2(i, j) + (inactive ? 0.0 : JTrad);
-    store_penetrating_shortwave(p, n, i, j, Itsw);
+    store_penetrating_shortwave<false>(p, n, Place{i, j, 0u}, Itsw);
     if (r.up_lw.p) r.up_lw.at2(i, j) = Iup;
     if (r.down_lw.p) r.down_lw.at2(i, j) = -Ila;
     if (r.down_sw.p) r.down_sw.at2(i, j) = -Itsw;
 }
 
 // One column of K2: freeze clamp, net-flux assembly and radiation.
-template <typename Real, bool TAU>
+template <typename Real, bool UNIT>
 __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const ne_params& p, const AtmosDev<Real>& a,
                                                         const double* __restrict__ afi,
                                                         const double* __restrict__ afj, const RadDev<Real>& rd,
                                                         const double* __restrict__ rfi,
                                                         const double* __restrict__ rfj, const View3<Real>& T,
-                                                        const View3<const Real>& S, const FluxOut& f,
-                                                        const NetOut& n, const RadOut& ro,
+                                                        const View3<const Real>& S, const NetOut& n, const RadOut& ro,
                                                         const View3<double>& frazil, double dt_frazil,
                                                         uint8_t* __restrict__ freeze_flags, double Qt,
                                                         double Qv, double Jv, double Ts_C, int i, int j) {
@@ -596,44 +612,33 @@ __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const 
         visit = flag != 0;
         if (visit) flag = 0;   // the stages only set flags
     }
+    const Place c2 = place<UNIT>(n.J_T, i, j);
     double dQ = visit ? freeze_column<Real>(g, p, T, S, i, j, dt_frazil) : 0.0;
-    if (frazil.p) frazil.at2(i, j) = dQ;
+    if (frazil.p) at<UNIT>(frazil, c2) = dQ;
 
-    Neighbours x = neighbours(afi[i], a.Nx, a.tx);
-    Neighbours y = neighbours(afj[j], a.Ny, a.ty);
-    double Jr = interp_field(a.rain, x, y, a.time);
-    double Js = interp_field(a.snow, x, y, a.time);
-    double rtx = 0.0, rty = 0.0, rtx_w = 0.0, rty_s = 0.0;   // τ here, or in the τ kernel after all columns
-    if (TAU) {
-        rtx = f.rtx.at2(i, j);
-        rty = f.rty.at2(i, j);
-        neighbour_momentum(g, f.rtx, f.rty, i, j, rtx_w, rty_s);
-    }
+    const Corners<UNIT> ca = corners<UNIT>(a.T, afi[i], a.Nx, a.tx, afj[j], a.Ny, a.ty);
+    double Jr = interp_at(a.rain, ca, a.time);
+    double Js = interp_at(a.snow, ca, a.time);
     bool inactive = !g.active(i, j, g.Nz - 1);
-    NetColumn c = assemble_column(g, p, Qt, Qv, Jv, rtx, rtx_w, rty, rty_s, Jr, Js, (double)T(i, j, g.Nz - 1),
-                                  inactive);
+    NetColumn c = assemble_column(g, p, Qt, Qv, Jv, 0.0, 0.0, 0.0, 0.0, Jr, Js, (double)T(i, j, g.Nz - 1),
+                                  inactive);   // τ in the τ kernel, after all columns
     double JT = c.J_T;
     if (p.radiation) {
-        Neighbours rx = neighbours(rfi[i], rd.Nx, rd.tx);
-        Neighbours ry = neighbours(rfj[j], rd.Ny, rd.ty);
-        double SW = interp_field(rd.sw, rx, ry, rd.time);
-        double LW = interp_field(rd.lw, rx, ry, rd.time);
+        const Corners<UNIT> cr = corners<UNIT>(rd.sw, rfi[i], rd.Nx, rd.tx, rfj[j], rd.Ny, rd.ty);
+        double SW = interp_at(rd.sw, cr, rd.time);
+        double LW = interp_at(rd.lw, cr, rd.time);
         double Iup, Ila, Itsw;
         double JTrad = radiation_column(p, Ts_C, SW, LW, Iup, Ila, Itsw);
         JT = JT + (inactive ? 0.0 : JTrad);
-        store_penetrating_shortwave(p, n, i, j, Itsw);
-        if (ro.up_lw.p) ro.up_lw.at2(i, j) = Iup;
-        if (ro.down_lw.p) ro.down_lw.at2(i, j) = -Ila;
-        if (ro.down_sw.p) ro.down_sw.at2(i, j) = -Itsw;
+        store_penetrating_shortwave<UNIT>(p, n, c2, Itsw);
+        if (ro.up_lw.p) at<UNIT>(ro.up_lw, c2) = Iup;
+        if (ro.down_lw.p) at<UNIT>(ro.down_lw, c2) = -Ila;
+        if (ro.down_sw.p) at<UNIT>(ro.down_sw, c2) = -Itsw;
     }
-    if (TAU) {
-        n.tau_x.at2(i, j) = c.tau_x;
-        n.tau_y.at2(i, j) = c.tau_y;
-    }
-    n.J_T.at2(i, j) = JT;
-    n.J_S.at2(i, j) = c.J_S;
-    n.J_w.at2(i, j) = c.J_w;
-    n.J_H.at2(i, j) = c.J_H;
+    at<UNIT>(n.J_T, c2) = JT;
+    at<UNIT>(n.J_S, c2) = c.J_S;
+    at<UNIT>(n.J_w, c2) = c.J_w;
+    at<UNIT>(n.J_H, c2) = c.J_H;
 }
 
 // K1 of the fused update_state: per column, interpolate the atmosphere and solve the fluxes,
@@ -643,7 +648,7 @@ __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const 
 // Defer (FP32 storage with parameters that take the FP32 iteration): a column whose FP32
 // iteration does not finish it is appended to `deferred` (count, then flattened columns) and left
 // to surface_deferred_kernel.
-template <typename Real, int PATH, bool Defer = false, int KBY = BY>
+template <typename Real, int PATH, bool UNIT, bool Defer = false, int KBY = BY>
 __global__ void __launch_bounds__(BX* KBY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __restrict__ fi,
                       const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
@@ -674,12 +679,12 @@ surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __
     r.deferred = false;
     bool inactive = true;
     if (in) {
-        r = surface_solve_column<Real, PATH, Defer>(tab, g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i,
+        r = surface_solve_column<Real, PATH, UNIT, Defer>(tab, g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i,
                                                             j, inactive);
         if (Defer && r.deferred)
             deferred[1 + atomicAdd(&deferred[0], 1)] = i + j * g.Nx;
         else
-            surface_finalize_column<Real, false>(g, p, a, fi, fj, rd, rfi, rfj, T, S, out, n, ro, frazil, dt_frazil,
+            surface_finalize_column<Real, UNIT>(g, p, a, fi, fj, rd, rfi, rfj, T, S, n, ro, frazil, dt_frazil,
                                                  freeze_flags, r.Qt, r.Qv, r.Jv, r.Ts_C, i, j);
     }
     bool solved = in && !inactive && !(Defer && r.deferred);
@@ -690,7 +695,7 @@ surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __
 // The columns surface_update_kernel deferred, finished as the kernel without deferral finishes
 // them (the FP32 iteration again, then the FP64 one): a grid-stride loop over the list, which is
 // empty in most steps. surface_tau_kernel, which runs after it, clears the count.
-template <typename Real, int PATH>
+template <typename Real, int PATH, bool UNIT>
 __global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 surface_deferred_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __restrict__ fi,
                         const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
@@ -710,9 +715,9 @@ surface_deferred_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* 
         if (q < count) {
             const int col = deferred[1 + q];
             const int i = col % g.Nx, j = col / g.Nx;
-            r = surface_solve_column<Real, PATH, false>(tab, g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i, j,
+            r = surface_solve_column<Real, PATH, UNIT, false>(tab, g, p, a, fi, fj, rd, rfi, rfj, cview(T), S, u, v, out, i, j,
                                                          inactive);
-            surface_finalize_column<Real, false>(g, p, a, fi, fj, rd, rfi, rfj, T, S, out, n, ro, frazil,
+            surface_finalize_column<Real, UNIT>(g, p, a, fi, fj, rd, rfi, rfj, T, S, n, ro, frazil,
                                                  dt_frazil, freeze_flags, r.Qt, r.Qv, r.Jv, r.Ts_C, i, j);
         }
         const bool solved = q < count && !inactive;
@@ -743,7 +748,7 @@ __global__ void __launch_bounds__(BX* BY) surface_tau_kernel(GridDev g, ne_param
 // FUSED (the step): each column then goes on as in the single model's K1 (freeze clamp of the
 // flagged columns, net fluxes other than τ, radiation); without it (the autotuner's timing
 // runs) the kernel only solves, leaving the state as it is.
-template <typename Real, int PATH, bool FUSED>
+template <typename Real, int PATH, bool UNIT, bool FUSED>
 __global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem* __restrict__ work, int nwork,
                            double dt_frazil, ne_counters* counters) {
@@ -767,11 +772,11 @@ batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkIt
         bool inactive = true;
         if (in)
         {
-            r = surface_solve_column<Real, PATH, false>(tab, g, rc.p, rc.a, rc.afi, rc.afj, rc.r, rc.rfi, rc.rfj, cview(rc.T),
+            r = surface_solve_column<Real, PATH, UNIT, false>(tab, g, rc.p, rc.a, rc.afi, rc.afj, rc.r, rc.rfi, rc.rfj, cview(rc.T),
                                                  cview(rc.S), rc.u, rc.v, rc.f, i, j, inactive);
             if (FUSED)
-                surface_finalize_column<Real, false>(g, rc.p, rc.a, rc.afi, rc.afj, rc.r, rc.rfi, rc.rfj, rc.T,
-                                                     cview(rc.S), rc.f, rc.n, rc.ro, rc.frazil, dt_frazil,
+                surface_finalize_column<Real, UNIT>(g, rc.p, rc.a, rc.afi, rc.afj, rc.r, rc.rfi, rc.rfj, rc.T,
+                                                     cview(rc.S), rc.n, rc.ro, rc.frazil, dt_frazil,
                                                      rc.freeze_flags, r.Qt, r.Qv, r.Jv, r.Ts_C, i, j);
         }
         if (in && !inactive) {
@@ -809,6 +814,72 @@ batch_surface_tau_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
+
+// Whether 2-D fields (null ones aside) share one layout: unit stride in i, one row stride, and less
+// than 4 GiB from the first value to the last.
+namespace {
+struct Layout2 {
+    int64_t sy = 0, sz = 0;
+    bool unit = true;
+    template <typename T>
+    void add(const View3<T>& v, int64_t rows, int64_t planes, int64_t esize) {
+        if (!v.p || !unit) return;
+        const bool first = sy == 0;
+        if (first) {
+            sy = v.sy;
+            sz = v.sz;
+        }
+        unit = v.sx == 1 && v.sy > 0 && v.sy == sy && (planes <= 1 || (v.sz > 0 && v.sz == sz)) &&
+               v.sy * rows * esize < ((int64_t)1 << 32);
+    }
+};
+
+// Runs f with the flux path and whether the fields are unit ones as compile-time constants.
+template <typename F>
+void with_path(int path, bool unit, F f) {
+    auto go = [&](auto u) {
+        switch (path) {
+        case 1: f(std::integral_constant<int, 1>{}, u); break;
+        case 2: f(std::integral_constant<int, 2>{}, u); break;
+        case 3: f(std::integral_constant<int, 3>{}, u); break;
+        case 4: f(std::integral_constant<int, 4>{}, u); break;
+        default: f(std::integral_constant<int, 0>{}, u); break;
+        }
+    };
+    if (unit) go(std::true_type{});
+    else go(std::false_type{});
+}
+}  // namespace
+
+// UNIT kernels' condition (Place, Corners): the 2-D outputs share one layout, the atmosphere's
+// fields another and the radiation's another, and the ocean's views have unit stride in i and span
+// less than 4 GiB. That is what a program that allocates its fields alike has; any other layout takes
+// the kernels with each view's own strides. About 30 views enter a column of K1, each with its own
+// strides in scalar registers (spilled and read back) and a 64-bit multiply-add per access; shared
+// offsets took K1 of 1440×560 from 173 to 158 µs (FP64) and from 92 to 83 (mixed), the exchange-state
+// solve of 360×180 from 44 to 42.
+template <typename Real>
+bool unit_fields(const GridDev& g, const AtmosDev<Real>& a, const RadDev<Real>& r, View3<const Real> T,
+                 View3<const Real> S, View3<const Real> u, View3<const Real> v, const FluxOut& f, const NetOut& n,
+                 const RadOut& ro, View3<double> frazil) {
+    Layout2 out, src, rad;
+    for (const View3<double>& x : {f.Qv, f.Qt, f.Jv, f.rtx, f.rty, f.us, f.ts, f.qs, f.Ts, n.tau_x, n.tau_y,
+                                  n.J_T, n.J_S, n.J_w, n.J_H, n.J_sw, ro.up_lw, ro.down_lw, ro.down_sw, frazil})
+        out.add(x, g.Ny, 1, 8);
+    out.add(f.iters, g.Ny, 1, 8);
+    for (const View3<const Real>* x : {&a.T, &a.u, &a.v, &a.q, &a.p, &a.rain, &a.snow}) src.add(*x, a.Ny, 2, sizeof(Real));
+    for (const View3<const Real>* x : {&r.sw, &r.lw}) rad.add(*x, r.Ny, 2, sizeof(Real));
+    bool ocean = true;
+    for (const View3<const Real>* x : {&T, &S, &u, &v})
+        ocean = ocean && x->sx == 1 && x->sy > 0 && x->sy * ((int64_t)g.Ny + 1) * (int64_t)sizeof(Real) < ((int64_t)1 << 32);
+    return out.unit && src.unit && rad.unit && ocean;
+}
+template bool unit_fields<double>(const GridDev&, const AtmosDev<double>&, const RadDev<double>&, View3<const double>,
+                                  View3<const double>, View3<const double>, View3<const double>, const FluxOut&,
+                                  const NetOut&, const RadOut&, View3<double>);
+template bool unit_fields<float>(const GridDev&, const AtmosDev<float>&, const RadDev<float>&, View3<const float>,
+                                 View3<const float>, View3<const float>, View3<const float>, const FluxOut&,
+                                 const NetOut&, const RadOut&, View3<double>);
 
 template <typename Real>
 AtmosDev<Real> atmos_dev(const ne_prescribed_atmosphere& a) {
@@ -944,15 +1015,21 @@ hipError_t launch_flux_solve_exchange(const GridDev& g, const ne_params& p, cons
     View3<const double> sw = view<const double>(a.downwelling_shortwave);
     View3<const double> lw = view<const double>(a.downwelling_longwave);
     const int path = flux_path(p);
-    auto kernel = path == 2   ? flux_solve_exchange_kernel<2>
-                  : path == 3 ? flux_solve_exchange_kernel<3>
-                  : path == 4 ? flux_solve_exchange_kernel<4>
-                  : path == 1 ? flux_solve_exchange_kernel<1>
-                              : flux_solve_exchange_kernel<0>;
-    hipLaunchKernelGGL(kernel, grid2d(g.Nx, g.Ny), dim3(BX, BY), 0, s, g, p, view<const double>(a.u),
-                       view<const double>(a.v), view<const double>(a.T), view<const double>(a.p),
-                       view<const double>(a.q), view<const double>(o.T), view<const double>(o.S),
-                       view<const double>(o.u), view<const double>(o.v), sw, lw, out, c);
+    const View3<const double> T = view<const double>(o.T), S = view<const double>(o.S), u = view<const double>(o.u),
+                              v = view<const double>(o.v);
+    Layout2 fields;
+    for (const View3<double>* x : {&out.Qv, &out.Qt, &out.Jv, &out.rtx, &out.rty, &out.us, &out.ts, &out.qs, &out.Ts})
+        fields.add(*x, g.Ny, 1, 8);
+    fields.add(out.iters, g.Ny, 1, 8);
+    for (const ne_view* x : {&a.u, &a.v, &a.T, &a.p, &a.q, &a.downwelling_shortwave, &a.downwelling_longwave})
+        fields.add(view<const double>(*x), g.Ny, 1, 8);
+    for (const View3<const double>* x : {&T, &S, &u, &v})
+        fields.unit = fields.unit && x->sx == 1 && x->sy > 0 && x->sy * ((int64_t)g.Ny + 1) * 8 < ((int64_t)1 << 32);
+    with_path(path, fields.unit, [&](auto P, auto U) {
+        hipLaunchKernelGGL((flux_solve_exchange_kernel<P(), U()>), grid2d(g.Nx, g.Ny), dim3(BX, BY), 0, s, g, p,
+                           view<const double>(a.u), view<const double>(a.v), view<const double>(a.T),
+                           view<const double>(a.p), view<const double>(a.q), T, S, u, v, sw, lw, out, c);
+    });
     if (g.ring) {
         auto ring = path == 2   ? flux_solve_ring_kernel<2>
                     : path == 3 ? flux_solve_ring_kernel<3>
@@ -1006,31 +1083,24 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
                                  hipStream_t s) {
     const int path = flux_path(p);
     const dim3 grid = grid2d(g.Nx, g.Ny);
-    if constexpr (sizeof(Real) == 4)
-    if (path >= 1 && path <= 3 && deferred && mixed_iteration_applies(p)) {
-        // the FP32 iteration alone at 6 wavefronts per SIMD in blocks of 8 rows, then the deferred
-        // columns
-        constexpr int KBY = NE_FLUX_MIXED_ROWS;
-        auto k1 = path == 2   ? surface_update_kernel<Real, 2, true, KBY>
-                  : path == 3 ? surface_update_kernel<Real, 3, true, KBY>
-                              : surface_update_kernel<Real, 1, true, KBY>;
-        auto k2 = path == 2   ? surface_deferred_kernel<Real, 2>
-                  : path == 3 ? surface_deferred_kernel<Real, 3>
-                              : surface_deferred_kernel<Real, 1>;
-        hipLaunchKernelGGL(k1, dim3((g.Nx + BX - 1) / BX, (g.Ny + KBY - 1) / KBY), dim3(BX, KBY), 0, s, g, p, a, fi, fj,
-                           r, rfi, rfj, T, S, u, v, out, n, ro, frazil, dt_frazil, freeze_flags, c, deferred);
-        const unsigned blocks = std::min<unsigned>(grid.x * grid.y, 256u);
-        hipLaunchKernelGGL(k2, dim3(blocks), dim3(BX, BY), 0, s, g, p, a, fi, fj, r, rfi, rfj, T, S, u, v, out, n, ro,
-                           frazil, dt_frazil, freeze_flags, c, deferred);
-        return hipGetLastError();
-    }
-    auto kernel = path == 2   ? surface_update_kernel<Real, 2>
-                  : path == 3 ? surface_update_kernel<Real, 3>
-                  : path == 4 ? surface_update_kernel<Real, 4>
-                  : path == 1 ? surface_update_kernel<Real, 1>
-                              : surface_update_kernel<Real, 0>;
-    hipLaunchKernelGGL(kernel, grid, dim3(BX, BY), 0, s, g, p, a, fi, fj, r, rfi, rfj, T, S, u, v, out, n, ro, frazil,
-                       dt_frazil, freeze_flags, c, (int*)nullptr);
+    const bool unit = unit_fields<Real>(g, a, r, cview(T), S, u, v, out, n, ro, frazil);
+    with_path(path, unit, [&](auto P, auto U) {
+        if constexpr (sizeof(Real) == 4 && P() >= 1 && P() <= 3)
+            if (deferred && mixed_iteration_applies(p)) {
+                // the FP32 iteration alone at 6 wavefronts per SIMD in blocks of 8 rows, then the
+                // deferred columns
+                constexpr int KBY = NE_FLUX_MIXED_ROWS;
+                hipLaunchKernelGGL((surface_update_kernel<Real, P(), U(), true, KBY>),
+                                   dim3((g.Nx + BX - 1) / BX, (g.Ny + KBY - 1) / KBY), dim3(BX, KBY), 0, s, g, p, a, fi,
+                                   fj, r, rfi, rfj, T, S, u, v, out, n, ro, frazil, dt_frazil, freeze_flags, c, deferred);
+                hipLaunchKernelGGL((surface_deferred_kernel<Real, P(), U()>), dim3(std::min<unsigned>(grid.x * grid.y, 256u)),
+                                   dim3(BX, BY), 0, s, g, p, a, fi, fj, r, rfi, rfj, T, S, u, v, out, n, ro, frazil,
+                                   dt_frazil, freeze_flags, c, deferred);
+                return;
+            }
+        hipLaunchKernelGGL((surface_update_kernel<Real, P(), U()>), grid, dim3(BX, BY), 0, s, g, p, a, fi, fj, r, rfi,
+                           rfj, T, S, u, v, out, n, ro, frazil, dt_frazil, freeze_flags, c, (int*)nullptr);
+    });
     return hipGetLastError();
 }
 template hipError_t launch_surface_update<double>(const GridDev&, const ne_params&, const AtmosDev<double>&,
@@ -1054,26 +1124,24 @@ hipError_t launch_surface_tau(const GridDev& g, const ne_params& p, const FluxOu
 
 template <typename Real>
 hipError_t launch_batch_surface_solve(const BatchRec<Real>* recs, const WorkItem* work, int nwork, int block,
-                                      int blocks, int path, bool fused, double dt_frazil, ne_counters* c,
+                                      int blocks, int path, bool unit, bool fused, double dt_frazil, ne_counters* c,
                                       hipStream_t s) {
     if (nwork <= 0) return hipSuccess;
     if (block <= 0 || block > BX * BY || (block & (block - 1)) != 0 || blocks <= 0) return hipErrorInvalidValue;
-    auto pick = [&](auto fused_tag) {
-        constexpr bool F = decltype(fused_tag)::value;
-        return path == 2   ? batch_surface_solve_kernel<Real, 2, F>
-               : path == 3 ? batch_surface_solve_kernel<Real, 3, F>
-               : path == 4 ? batch_surface_solve_kernel<Real, 4, F>
-               : path == 1 ? batch_surface_solve_kernel<Real, 1, F>
-                           : batch_surface_solve_kernel<Real, 0, F>;
-    };
-    auto kernel = fused ? pick(std::true_type{}) : pick(std::false_type{});
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(block), 0, s, recs, work, nwork, dt_frazil, c);
+    with_path(path, unit, [&](auto P, auto U) {
+        if (fused)
+            hipLaunchKernelGGL((batch_surface_solve_kernel<Real, P(), U(), true>), dim3(blocks), dim3(block), 0, s, recs,
+                               work, nwork, dt_frazil, c);
+        else
+            hipLaunchKernelGGL((batch_surface_solve_kernel<Real, P(), U(), false>), dim3(blocks), dim3(block), 0, s, recs,
+                               work, nwork, dt_frazil, c);
+    });
     return hipGetLastError();
 }
 template hipError_t launch_batch_surface_solve<double>(const BatchRec<double>*, const WorkItem*, int, int, int, int,
-                                                       bool, double, ne_counters*, hipStream_t);
+                                                       bool, bool, double, ne_counters*, hipStream_t);
 template hipError_t launch_batch_surface_solve<float>(const BatchRec<float>*, const WorkItem*, int, int, int, int,
-                                                      bool, double, ne_counters*, hipStream_t);
+                                                      bool, bool, double, ne_counters*, hipStream_t);
 
 template <typename Real>
 hipError_t launch_batch_surface_tau(const BatchRec<Real>* recs, const WorkItem* work, int nwork, int block,
