@@ -62,11 +62,11 @@ constexpr int TC = 63;            // cells per tile row
 #ifndef NE_STAGE_WAVES_PER_EU_F64
 #define NE_STAGE_WAVES_PER_EU_F64 4
 #endif
-template <typename Real, bool TWO_COLOR, bool LAST>
-constexpr int stage_waves() {
+template <typename Real>
+constexpr int stage_waves(bool two_color, bool last) {
     return sizeof(Real) == 8 ? NE_STAGE_WAVES_PER_EU_F64
-           : TWO_COLOR       ? NE_STAGE_WAVES_PER_EU_F32_TWO_COLOR
-           : LAST            ? NE_STAGE_WAVES_PER_EU_F32_LAST
+           : two_color       ? NE_STAGE_WAVES_PER_EU_F32_TWO_COLOR
+           : last            ? NE_STAGE_WAVES_PER_EU_F32_LAST
                              : NE_STAGE_WAVES_PER_EU_F32;
 }
 constexpr int PLAIN_TR = NE_PLAIN_TR;  // cell rows per tile of the single-model kernel
@@ -90,10 +90,15 @@ struct TileShared {
 __host__ __device__ inline int tiles_x(int Nx) { return (Nx + TC - 1) / TC; }
 __host__ __device__ inline int tiles_y(int Ny, int tr) { return (Ny + tr - 1) / tr; }
 
-// Blocks of the single-model kernel: every tile's levels in chunks of `levels`.
-inline int grid_blocks(const GridDev& g, int levels) {
-    int n = tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR);
-    return ((n + NXCD - 1) / NXCD) * NXCD * level_chunks(g.Nz, levels);
+// How the single-model kernel cuts its tiles' levels: tiles 0 … first-1 in chunks of `levels`, the
+// others in chunks of `rest_levels` (stage_plan).
+struct StagePlan {
+    int tiles, first, levels, rest_levels;
+    __host__ __device__ int first_per_xcd() const { return (first + NXCD - 1) / NXCD; }
+    __host__ __device__ int rest_per_xcd() const { return (tiles - first + NXCD - 1) / NXCD; }
+};
+inline int grid_blocks(const StagePlan& p, int Nz) {
+    return NXCD * (p.first_per_xcd() * level_chunks(Nz, p.levels) + p.rest_per_xcd() * level_chunks(Nz, p.rest_levels));
 }
 
 // Face order at level k from the three thresholds of its stencil: the face is
@@ -561,24 +566,33 @@ __device__ __forceinline__ void tile_body(TileShared<Real, TR>& sh, const GridDe
 
 // Single model: one block per tile and chunk of levels, ordered so that each XCD (blocks are dealt
 // round-robin to the 8 XCDs) receives a contiguous band of tiles, its uppermost chunks first: they
-// hold the most active cells, and the short blocks of the lower chunks fill the launch's tail.
+// hold the most active cells, and the short blocks of the lower chunks, and of the tiles cut into
+// shorter ones, fill the launch's tail.
 template <typename Real, int MODE, bool TWO_COLOR, bool WATCH = false, bool BEER = false>
 __global__ void __launch_bounds__(TW * PLAIN_TR)
-__attribute__((amdgpu_waves_per_eu(stage_waves<Real, TWO_COLOR, WATCH && MODE == 0>())))
+__attribute__((amdgpu_waves_per_eu(stage_waves<Real>(TWO_COLOR, WATCH && MODE == 0))))
 tracer_tile_kernel(GridDev g, TracerLayout L, const Real* u, const Real* v, const Real* w, const Real* T0,
                    const Real* S0, const Real* Tin, const Real* Sin, Real* Tout, Real* Sout, const double* JT,
-                   const double* JS, const double* Jw, TracerForcing F, double beta_dt, int levels, int stochastic,
+                   const double* JS, const double* Jw, TracerForcing F, double beta_dt, StagePlan plan, int stochastic,
                    uint32_t seed) {
     __shared__ TileShared<Real, PLAIN_TR> sh;
-    const int ntx = tiles_x(g.Nx), nty = tiles_y(g.Ny, PLAIN_TR);
-    const int nch = level_chunks(g.Nz, levels);
-    const int ntiles = ntx * nty;
-    const int per = (ntiles + NXCD - 1) / NXCD;
-    const int q = (int)(blockIdx.x / NXCD) % per;
-    const int chunk = nch - 1 - (int)(blockIdx.x / NXCD) / per;
-    const int tile = (int)(blockIdx.x % NXCD) * per + q;
-    if (tile >= ntiles) return;
-    if (F.residual) F.residual += RESIDUAL_SLOT * (tile * nch + chunk);   // this chunk's totals
+    const int ntx = tiles_x(g.Nx), x = (int)(blockIdx.x % NXCD);
+    int q = (int)(blockIdx.x / NXCD);
+    int nch = level_chunks(g.Nz, plan.levels), per = plan.first_per_xcd(), end = plan.first, levels = plan.levels;
+    int tile = 0, slot = 0;
+    if (q >= per * nch) {   // the tiles cut into shorter chunks
+        q -= per * nch;
+        tile = plan.first;
+        slot = plan.first * nch;
+        levels = plan.rest_levels;
+        nch = level_chunks(g.Nz, levels);
+        per = plan.rest_per_xcd();
+        end = plan.tiles;
+    }
+    const int t = x * per + q % per, chunk = nch - 1 - q / per;
+    tile += t;
+    if (tile >= end) return;
+    if (F.residual) F.residual += RESIDUAL_SLOT * (slot + t * nch + chunk);   // this chunk's totals
     const int k0 = chunk * levels;
     tile_body<Real, MODE, PLAIN_TR, TWO_COLOR, WATCH, BEER>(sh, g, L, u, v, w, T0, S0, Tin, Sin, Tout, Sout, JT, JS, Jw, F,
                                                      beta_dt, (tile % ntx) * TC, (tile / ntx) * PLAIN_TR, k0,
@@ -591,7 +605,7 @@ tracer_tile_kernel(GridDev g, TracerLayout L, const Real* u, const Real* v, cons
 // stage 1: T¹ = T + β₁Δt G(T); stage 2: T² = T + β₂Δt G(T¹); stage 3: T = T + β₃Δt G(T²).
 template <typename Real, int TR, bool TWO_COLOR, bool WATCH>
 __global__ void __launch_bounds__(TW * TR)
-__attribute__((amdgpu_waves_per_eu(stage_waves<Real, TWO_COLOR, WATCH>())))
+__attribute__((amdgpu_waves_per_eu(stage_waves<Real>(TWO_COLOR, WATCH))))
 batch_stage_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem* __restrict__ work, int nwork,
                    int stage, double beta_dt) {
     __shared__ TileShared<Real, TR> sh;
@@ -861,6 +875,47 @@ TracerLayout host_layout(const View3<const Real>& c, const View3<const Real>& u,
     return L;
 }
 
+// Levels of one block. A block takes its levels in series, about 2.7 µs each when the chip is not
+// full, so a grid (or batch) of few tiles has each tile's column cut into chunks until there are
+// about NE_STAGE_TARGET_BLOCKS blocks; every chunk pays the tile's set-up and one more z face
+// (≈ 1.5 levels), so full grids are not cut. 1024 blocks of the FP64 kernel are resident at once;
+// 1536 measured best over 768 … 3072 (whole steps, uncut → cut, µs: one column of 50 levels
+// 166 → 57, 90×40×10 139 → 89, 353×137×19 mixed 235 → 142, 481×187×23 578 → 485, 12 uneven FP64
+// members 448 → 362 and mixed ones 295 → 122; 1440×560×10 has 3220 tiles and stays uncut: two chunks
+// per tile took its FP64 stage from 136 to 151 µs).
+#ifndef NE_STAGE_TARGET_BLOCKS
+#define NE_STAGE_TARGET_BLOCKS 1536
+#endif
+int64_t stage_tile_levels(const GridDev& g) { return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR) * g.Nz; }
+
+int stage_levels(const GridDev& g, int64_t tile_levels) {
+    const int64_t wanted = std::max<int64_t>((tile_levels + NE_STAGE_TARGET_BLOCKS - 1) / NE_STAGE_TARGET_BLOCKS, 1);
+    const int chunks = (int)((g.Nz + wanted - 1) / wanted);
+    return (g.Nz + chunks - 1) / chunks;
+}
+
+namespace {
+// The chip holds `waves` 4-wavefront blocks of a stage kernel per CU at once. A launch of more tiles
+// than that ends with a partly filled round of whole columns, so the tiles left over from full rounds
+// are cut into as many chunks as have a place in one (each chunk costs a set-up of about 1½ levels,
+// which the idle places pay). 1440×560×10 has 3220 tiles: 148 are left over from 3 rounds of 1024
+// (FP64), or from 2 of 1536 (the mixed form's last stage), and the stages took 128 against 132 µs and
+// 91 against 93; from 1 of 1792 (its other stages) 1428 are, more than half a round, and stay whole.
+// Cutting 256 or 1024 tiles more took the FP64 stage to 130 and 134 µs. Grids of fewer tiles than
+// places are cut throughout (stage_levels).
+constexpr int CUS = 256;
+StagePlan stage_plan(const GridDev& g, int waves) {
+    const int tiles = tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR), places = waves * CUS;
+    if (tiles < places) {
+        const int levels = stage_levels(g, stage_tile_levels(g));
+        return {tiles, tiles, levels, levels};
+    }
+    const int rest = tiles % places;
+    const int chunks = rest > 0 ? std::min(places / rest, g.Nz) : 1;
+    return {tiles, chunks > 1 ? tiles - rest : tiles, g.Nz, (g.Nz + chunks - 1) / chunks};
+}
+}  // namespace
+
 template <typename Real>
 hipError_t launch_rk_stage(const GridDev& g, View3<const Real> u, View3<const Real> v, View3<const Real> w,
                            View3<const Real> T0, View3<const Real> S0, View3<const Real> Tin, View3<const Real> Sin,
@@ -868,35 +923,35 @@ hipError_t launch_rk_stage(const GridDev& g, View3<const Real> u, View3<const Re
                            View3<const double> Jw, TracerForcing forcing, double beta_dt, bool stochastic,
                            double time, hipStream_t s) {
     TracerLayout L = host_layout<Real>(Tin, u, v, w, JT);
-    const int levels = stage_levels(g, stage_tile_levels(g));
-    const dim3 grid(grid_blocks(g, levels)), block(TW, PLAIN_TR);
+    const bool watch = forcing.freeze_flags != nullptr;
+    const StagePlan plan = stage_plan(g, stage_waves<Real>(forcing.two_color != 0, watch));
+    const dim3 grid(grid_blocks(plan, g.Nz)), block(TW, PLAIN_TR);
     const int sr = stochastic ? 1 : 0;
     const uint32_t seed = step_seed(time);
-    const bool watch = forcing.freeze_flags != nullptr;
     const bool beer = forcing.beer != nullptr;   // a model's factors (per-phase calls compute them)
     if (forcing.two_color && watch && beer)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, true, true>), grid, block, 0, s, g, L, u.p, v.p, w.p,
-                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, plan,
                            sr, seed);
     else if (forcing.two_color && beer)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, false, true>), grid, block, 0, s, g, L, u.p, v.p, w.p,
-                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           T0.p, S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, plan,
                            sr, seed);
     else if (forcing.two_color && watch)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, true>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, plan,
                            sr, seed);
     else if (forcing.two_color)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, true, false>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, plan,
                            sr, seed);
     else if (watch)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, false, true>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, plan,
                            sr, seed);
     else
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 0, false, false>), grid, block, 0, s, g, L, u.p, v.p, w.p, T0.p,
-                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, levels,
+                           S0.p, Tin.p, Sin.p, Tout.p, Sout.p, JT.p, JS.p, Jw.p, forcing, beta_dt, plan,
                            sr, seed);
     return hipGetLastError();
 }
@@ -954,14 +1009,14 @@ hipError_t launch_tendency(const GridDev& g, View3<const Real> u, View3<const Re
                            View3<const double> JS, View3<const double> Jw, TracerForcing forcing, View3<Real> GT,
                            View3<Real> GS, hipStream_t s) {
     TracerLayout L = host_layout<Real>(T, u, v, w, JT);
-    const int levels = stage_levels(g, stage_tile_levels(g));
-    const dim3 grid(grid_blocks(g, levels)), block(TW, PLAIN_TR);
+    const StagePlan plan = stage_plan(g, stage_waves<Real>(forcing.two_color != 0, false));
+    const dim3 grid(grid_blocks(plan, g.Nz)), block(TW, PLAIN_TR);
     if (forcing.two_color)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 1, true>), grid, block, 0, s, g, L, u.p, v.p, w.p, T.p, S.p, T.p,
-                           S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0, levels, 0, 0u);
+                           S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0, plan, 0, 0u);
     else
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 1, false>), grid, block, 0, s, g, L, u.p, v.p, w.p, T.p, S.p,
-                           T.p, S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0, levels, 0, 0u);
+                           T.p, S.p, GT.p, GS.p, JT.p, JS.p, Jw.p, forcing, 0.0, plan, 0, 0u);
     return hipGetLastError();
 }
 template hipError_t launch_tendency<double>(const GridDev&, View3<const double>, View3<const double>,
@@ -1028,32 +1083,18 @@ int64_t budget_blocks(const GridDev& g) {
     return (int64_t)gr.x * gr.y;
 }
 
-// The kernels of launch_budget with the partials in the device's `scratch` array; allocates
-// nothing. Every block overwrites its own pair, so nothing needs clearing between calls.
-// One slot of 4 doubles per tile and chunk of levels of the tiling with the most tiles (the fewest
-// rows: the single-model tiling or the batch's 4-row one); a batch of taller tiles uses the first
-// slots.
+// One slot of 4 doubles per block of the FP32 state's last stage: the single-model kernel's, or the
+// batch's of its 4-row tiles with no shorter chunks than the grid alone would have (taller tiles use
+// the first slots).
 int64_t residual_slots(const GridDev& g) {
-    return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR < 4 ? PLAIN_TR : 4) * level_chunks(g.Nz, stage_levels(g, stage_tile_levels(g)));
-}
-
-// Levels of one block. A block takes its levels in series, about 2.7 µs each when the chip is not
-// full, so a grid (or batch) of few tiles has each tile's column cut into chunks until there are
-// about NE_STAGE_TARGET_BLOCKS blocks; every chunk pays the tile's set-up and one more z face
-// (≈ 1.5 levels), so full grids are not cut. 1024 blocks of the FP64 kernel are resident at once;
-// 1536 measured best over 768 … 3072 (whole steps, uncut → cut, µs: one column of 50 levels
-// 166 → 57, 90×40×10 139 → 89, 353×137×19 mixed 235 → 142, 481×187×23 578 → 485, 12 uneven FP64
-// members 448 → 362 and mixed ones 295 → 122; 1440×560×10 has 3220 tiles and stays uncut: two chunks
-// per tile took its FP64 stage from 136 to 151 µs).
-#ifndef NE_STAGE_TARGET_BLOCKS
-#define NE_STAGE_TARGET_BLOCKS 1536
-#endif
-int64_t stage_tile_levels(const GridDev& g) { return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR) * g.Nz; }
-
-int stage_levels(const GridDev& g, int64_t tile_levels) {
-    const int64_t wanted = std::max<int64_t>((tile_levels + NE_STAGE_TARGET_BLOCKS - 1) / NE_STAGE_TARGET_BLOCKS, 1);
-    const int chunks = (int)((g.Nz + wanted - 1) / wanted);
-    return (g.Nz + chunks - 1) / chunks;
+    int64_t n = (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR < 4 ? PLAIN_TR : 4) *
+                level_chunks(g.Nz, stage_levels(g, stage_tile_levels(g)));
+    for (bool two_color : {false, true}) {
+        const StagePlan p = stage_plan(g, stage_waves<float>(two_color, true));
+        n = std::max<int64_t>(n, (int64_t)p.first * level_chunks(g.Nz, p.levels) +
+                                     (int64_t)(p.tiles - p.first) * level_chunks(g.Nz, p.rest_levels));
+    }
+    return n;
 }
 
 hipError_t launch_residual_reduce(const double* residual, const GridDev& g, double* out, hipStream_t s) {
@@ -1061,6 +1102,8 @@ hipError_t launch_residual_reduce(const double* residual, const GridDev& g, doub
     return hipGetLastError();
 }
 
+// The kernels of launch_budget with the partials in the device's `scratch` array; allocates
+// nothing. Every block overwrites its own pair, so nothing needs clearing between calls.
 hipError_t launch_budget_noalloc(double* partial, const GridDev& g, View3<const double> c, double weight,
                                  double* out, hipStream_t s) {
     const dim3 gr = grid2d(g.Nx, g.Ny);

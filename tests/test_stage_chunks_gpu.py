@@ -28,3 +28,18 @@ def test_chunked_stages_match_the_oracle(require_gpu, Nx, Ny, Nz, topology_x, st
     assert_rel(gm.T.cpu().numpy(), om.T, 1e-12, "T")
     assert_rel(gm.S.cpu().numpy(), om.S, 1e-12, "S")
     gm.close()
+
+
+# 1133 and 1144 tiles of 63×4 cells: more than the 1024 blocks the chip holds, so that the last 109 (120)
+# tiles alone are cut, into chunks of one level, and of two with a last one of one
+@pytest.mark.parametrize("Nx,Ny,Nz", [(640, 410, 4), (690, 416, 15)])
+def test_stages_of_more_tiles_than_places_match_the_oracle(require_gpu, Nx, Ny, Nz):
+    from numericalearth_hip.model import OceanOnlyModel
+    case = make_case(Nx, Ny, Nz, seed=12, topology_x=NE_PERIODIC, longitude=(0.0, 360.0), sigma_cells=6.0, n_times=2)
+    om = O.OracleModel(case).reconcile()
+    gm = OceanOnlyModel(case)
+    om.time_step(1200.0)
+    gm.time_step(1200.0)
+    assert_rel(gm.T.cpu().numpy(), om.T, 1e-12, "T")
+    assert_rel(gm.S.cpu().numpy(), om.S, 1e-12, "S")
+    gm.close()
