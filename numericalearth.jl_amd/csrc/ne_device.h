@@ -1335,13 +1335,12 @@ __device__ __forceinline__ Corners<UNIT> corners(const View3<const Real>& layout
     }
     return c;
 }
-// interp_field at such corners: the same operations.
+// interp_field at such corners, of a field that is there: the same operations.
 template <bool UNIT, typename Real>
 __device__ __forceinline__ double interp_at(const View3<const Real>& d, const Corners<UNIT>& c, const ne_time_interp& t) {
     if constexpr (!UNIT) {
         return interp_field(d, c.x, c.y, t);
     } else {
-        if (d.p == nullptr) return 0.0;
         const double xi = c.x.w, eta = c.y.w;
         const double w00 = (1.0 - xi) * (1.0 - eta), w01 = (1.0 - xi) * eta, w10 = xi * (1.0 - eta), w11 = xi * eta;
         auto value = [](const Real* base, uint32_t o) {
