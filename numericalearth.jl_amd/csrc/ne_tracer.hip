@@ -682,6 +682,10 @@ constexpr int BY = 4;
 
 inline dim3 grid2d(int Nx, int Ny) { return dim3((Nx + BX - 1) / BX, (Ny + BY - 1) / BY); }
 
+// The levels of a column whose values are loaded before the first is added: level by level each
+// addition waited a memory latency for its value (719×281×17 FP64: 10.2 µs, with 2, 4, 5 and 10 levels
+// 9.3, 8.7, 8.9 and 9.7).
+constexpr int LOAD_LEVELS = 4;
 template <typename Real>
 __global__ void budget_partial_kernel(GridDev g, View3<const Real> c, double weight, double* partial) {
     __shared__ double ss[BX * BY], sc[BX * BY];
@@ -691,10 +695,20 @@ __global__ void budget_partial_kernel(GridDev g, View3<const Real> c, double wei
     DD acc = {0.0, 0.0};
     if (i < g.Nx && j < g.Ny) {
         int k0 = g.kmin[i + (int64_t)j * g.Nx];
-        for (int k = k0; k < g.Nz; k++) {
-            double x = weight * (g.Az[j] * g.dz[k]) * (double)c(i, j, k);
-            DD xd = {x, 0.0};
-            acc = dd_add(acc, xd);
+        const double Az = g.Az[j];
+        for (int kb = 0; kb < g.Nz; kb += LOAD_LEVELS) {
+            if (!__any(kb + LOAD_LEVELS > k0)) continue;   // no active cell of the wavefront
+            double value[LOAD_LEVELS];
+#pragma unroll
+            for (int l = 0; l < LOAD_LEVELS; l++)   // levels past the top: the top one's, not used
+                value[l] = (double)c(i, j, min(kb + l, g.Nz - 1));
+#pragma unroll
+            for (int l = 0; l < LOAD_LEVELS; l++) {
+                if (kb + l >= g.Nz || kb + l < k0) continue;
+                double x = weight * (Az * g.dz[kb + l]) * value[l];
+                DD xd = {x, 0.0};
+                acc = dd_add(acc, xd);
+            }
         }
     }
     ss[t] = acc.s;
