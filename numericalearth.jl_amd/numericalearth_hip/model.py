@@ -261,7 +261,8 @@ class OceanOnlyModel:
         h = C.c_void_p()
         check(self.lib.ne_model_create(self.ctx.handle, C.byref(d), C.byref(h), s), "ne_model_create")
         self.handle = h
-        self._budget_out = torch.zeros(2, dtype=f64, device=dev)
+        # pinned host memory, which the budget kernel writes itself: a wait for its stream in place of a copy back
+        self._budget_out = torch.zeros(2, dtype=f64, pin_memory=True)
         self.streams = {}
         for which, series, fields in ((0, "atmosphere", self.atm), (1, "radiation", self.rad)):
             if series in resident:
@@ -320,6 +321,7 @@ class OceanOnlyModel:
         fn = self.lib.ne_budget_f64 if field.dtype == torch.float64 else self.lib.ne_budget_f32
         check(fn(self.ctx.handle, C.byref(self.grid.struct), torch_view(field), float(weight),
                  self._budget_out.data_ptr(), stream_handle(stream)), "ne_budget")
+        (stream if stream is not None else torch.cuda.current_stream()).synchronize()
         s, c = self._budget_out.tolist()
         return s + c
 
