@@ -13,16 +13,11 @@ namespace ne {
 
 namespace {
 
+// Rows of a block: the wavefronts that share one copy of the stability table. K1 with 8, 4, 2 rows takes
+// 76, 75.5, 78 µs at 1440×560 and 24.9, 22.7, 22.7 at 353×137 (mixed form), with 4, 2, 1 rows 169, 182,
+// 247 at 1440×560 and 31.5 throughout at 90×40 (FP64).
 constexpr int BX = 64;
 constexpr int BY = 4;
-// Rows of the deferring K1's blocks (the mixed form's FP32 iteration). Its columns are cheap, and
-// blocks of 8 rows halve what each column pays of the block's fixed work (the column sort, the
-// counters' reduction, the launch): 158 → 125 µs at 1440×560×10 against 4 rows, and 263 µs
-// with 2 (same-box A/B; the FP64 K1 is 2 % slower with 8). A power of two.
-#ifndef NE_FLUX_MIXED_ROWS
-#define NE_FLUX_MIXED_ROWS 8
-#endif
-
 // Minimum wavefronts per SIMD requested for the flux-solve kernels (bounds their VGPRs).
 #ifndef NE_FLUX_WAVES_PER_EU
 #define NE_FLUX_WAVES_PER_EU 4
@@ -684,18 +679,18 @@ __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const 
 // Defer (FP32 storage with parameters that take the FP32 iteration): a column whose FP32
 // iteration does not finish it is appended to `deferred` (count, then flattened columns) and left
 // to surface_deferred_kernel.
-template <typename Real, int PATH, bool UNIT, bool Defer = false, int KBY = BY>
-__global__ void __launch_bounds__(BX* KBY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
+template <typename Real, int PATH, bool UNIT, bool Defer = false>
+__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
 surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __restrict__ fi,
                       const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
                       const double* __restrict__ rfj, View3<Real> T, View3<const Real> S, View3<const Real> u,
                       View3<const Real> v, FluxOut out, NetOut n, RadOut ro, View3<double> frazil, double dt_frazil,
                       uint8_t* __restrict__ freeze_flags, ne_counters* counters, int* deferred) {
     __shared__ FluxTable<Real, PATH> tab;
-    TableLoad<BX * KBY, FluxTable<Real, PATH>> table;
+    TableLoad<BX * BY, FluxTable<Real, PATH>> table;
     table.load();
     int i = blockIdx.x * BX + threadIdx.x;
-    int j = blockIdx.y * KBY + threadIdx.y;
+    int j = blockIdx.y * BY + threadIdx.y;
     if (out.iters.p && (PATH == 0 || PATH == 4)) {
         // Columns of the block in order of the iteration count the previous solve took, the
         // stable ones last (solve_order_key): the fixed point runs until the slowest column of a
@@ -707,9 +702,9 @@ surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __
         const int t = threadIdx.x + threadIdx.y * BX;
         const bool own = i < g.Nx && j < g.Ny;
         const int key = own ? solve_order_key(out, i, j) : SORT_BINS - 1;
-        const int c = sorted_block_column<BX * KBY>(key, t);
+        const int c = sorted_block_column<BX * BY>(key, t);
         i = blockIdx.x * BX + c % BX;
-        j = blockIdx.y * KBY + c / BX;
+        j = blockIdx.y * BY + c / BX;
     }
     const bool in = i < g.Nx && j < g.Ny;
     // a work-item outside the grid reads the last column or row, without a branch around the loads
@@ -1133,11 +1128,8 @@ hipError_t launch_surface_update(const GridDev& g, const ne_params& p, const Atm
     with_path(path, unit, [&](auto P, auto U) {
         if constexpr (sizeof(Real) == 4 && P() >= 1 && P() <= 3)
             if (deferred && mixed_iteration_applies(p)) {
-                // the FP32 iteration alone at 6 wavefronts per SIMD in blocks of 8 rows, then the
-                // deferred columns
-                constexpr int KBY = NE_FLUX_MIXED_ROWS;
-                hipLaunchKernelGGL((surface_update_kernel<Real, P(), U(), true, KBY>),
-                                   dim3((g.Nx + BX - 1) / BX, (g.Ny + KBY - 1) / KBY), dim3(BX, KBY), 0, s, g, p, a, fi,
+                // the FP32 iteration alone, then the deferred columns
+                hipLaunchKernelGGL((surface_update_kernel<Real, P(), U(), true>), grid, dim3(BX, BY), 0, s, g, p, a, fi,
                                    fj, r, rfi, rfj, T, S, u, v, out, n, ro, frazil, dt_frazil, freeze_flags, c, deferred);
                 hipLaunchKernelGGL((surface_deferred_kernel<Real, P(), U()>), dim3(std::min<unsigned>(grid.x * grid.y, 256u)),
                                    dim3(BX, BY), 0, s, g, p, a, fi, fj, r, rfi, rfj, T, S, u, v, out, n, ro, frazil,
