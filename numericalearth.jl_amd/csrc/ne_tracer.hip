@@ -46,10 +46,10 @@ constexpr int TC = 63;            // cells per tile row
 // Minimum wavefronts per SIMD requested for the stage kernels. The software pipeline holds
 // the next level's inputs in registers, and a spilled register defeats it (a reload from
 // scratch waits for every load in flight), so the targets are the largest occupancies whose
-// register budget fits without spills, measured on 1440×560×10: FP64 4 (≈116–125 VGPRs;
-// 5 spills and runs 30 % slower), FP32 7 (≤ 72 VGPRs, a 12-byte spill, faster than 5 or 6)
-// and 5 for the FP32 instances with the two-colour forcing (≈ 93 VGPRs). The FP32 state's last
-// stage, which forms its update in FP64, takes 6 (≤ 80 VGPRs).
+// register budget holds the pipeline, measured on 1440×560×10: FP64 4 (≤ 128 VGPRs; 5 spills and runs
+// 30 % slower), FP32 7 (72 VGPRs, faster than 5 or 6) and 5 for the FP32 instances with the two-colour
+// forcing (≤ 96 VGPRs). The FP32 state's last stage, which forms its update in FP64, takes 6
+// (80 VGPRs, 6 of them spilled).
 #ifndef NE_STAGE_WAVES_PER_EU_F32
 #define NE_STAGE_WAVES_PER_EU_F32 7
 #endif
