@@ -638,19 +638,37 @@ __host__ inline bool default_surface_constants(const ne_params& p) {
     return memcmp(&q, &p, sizeof q) == 0;
 }
 
-// True when the iteration may take the logarithm of every quantity it forms (flux path 3): the
-// Edson roughness lengths with positive constants, and a gustiness that keeps u★ above zero.
+// True when the iteration may take the logarithm of every quantity it forms (flux path 3, LogForm in
+// flux_column): the Edson roughness lengths, convective gustiness, and constants within ranges that hold
+// every physical set (the defaults lie near the middle of each) and in which that form's shortcuts are
+// exact or round as its comments say. Any other set takes path 1, which has none of them.
 __host__ inline bool positive_surface_constants(const ne_params& p) {
-    const double positive[] = {p.von_karman_constant, p.minimum_gustiness, p.roughness_gravitational_acceleration,
-                               p.air_kinematic_viscosity, p.charnock_parameter + p.smooth_wall_parameter,
-                               p.maximum_momentum_roughness, p.reynolds_scaling_A, p.maximum_scalar_roughness,
-                               p.surface_layer_height - p.zero_plane_displacement};
-    for (double x : positive)
-        if (!(x >= 1e-30 && x <= 1e30)) return false;
-    const double zero_or_positive[] = {p.gustiness_parameter, p.charnock_parameter, p.smooth_wall_parameter,
-                                       p.boundary_layer_height, fabs(p.reynolds_scaling_b)};
-    for (double x : zero_or_positive)
-        if (!(x >= 0.0 && x <= 1e30)) return false;
+    const struct {
+        double value, least, largest;
+    } ranges[] = {
+        {p.von_karman_constant, 0.1, 1.0},
+        // the gustiness w = β∛x is taken as 0 for x < 10⁻³⁰, where it is at most 100·10⁻¹⁰ and the
+        // maximum with the minimum gustiness keeps 10⁻⁴ or more; and x = −u★b★h stays far below 2¹²⁸
+        {p.minimum_gustiness, 1e-4, 1e2},
+        {p.gustiness_parameter, 0.0, 1e2},
+        {p.boundary_layer_height, 0.0, 1e5},
+        // log R★ and the other logarithms lie within ±100, so the exponential of −b·log R★ is far from
+        // its limits (ne_exp: ±700) and ℓq and log ℓq agree; sums of logarithms keep their relative
+        // accuracy
+        {p.roughness_gravitational_acceleration, 0.1, 1e3},
+        {p.air_kinematic_viscosity, 1e-7, 1e-3},
+        {p.charnock_parameter, 0.0, 1.0},
+        {p.smooth_wall_parameter, 0.0, 1e1},
+        {p.charnock_parameter + p.smooth_wall_parameter, 1e-4, 11.0},
+        {p.maximum_momentum_roughness, 1e-4, 1e2},
+        {p.reynolds_scaling_A, 1e-8, 0.1},
+        {p.reynolds_scaling_b, -4.0, 4.0},
+        {p.maximum_scalar_roughness, 1e-8, 1e1},
+        {p.surface_layer_height - p.zero_plane_displacement, 0.1, 1e3},
+        {p.mesoscale_gustiness ? p.mesoscale_velocity : 0.0, -1e3, 1e3},
+    };
+    for (const auto& r : ranges)
+        if (!(r.value >= r.least && r.value <= r.largest)) return false;
     return p.convective_gustiness && p.momentum_roughness == NE_ROUGHNESS_EDSON &&
            p.temperature_roughness == NE_ROUGHNESS_EDSON && p.water_vapor_roughness == NE_ROUGHNESS_EDSON;
 }
@@ -1137,9 +1155,10 @@ __device__ __forceinline__ ColumnFluxes flux_column(const Tab& tab, const ne_par
             double Usg2;
             if constexpr (LogForm) {
                 // the convective gustiness with ne_cbrt_ge1's first value and Halley step, valid for
-                // any x in FP32's normal range: below 10⁻³⁰, β∛x is far under the minimum
-                // gustiness the maximum keeps, so x is taken as 0 there. Minima and maxima are plain
-                // selects here: a NaN of the iterate reaches all three scales through u★ or 1/L
+                // any x in FP32's normal range: below 10⁻³⁰, β∛x is under the minimum gustiness the
+                // maximum keeps (the ranges of positive_surface_constants), so x is taken as 0 there.
+                // Minima and maxima are plain selects here: a NaN of the iterate reaches all three
+                // scales through u★ or 1/L
                 const double Jb = -us * bstar;
                 const double x = (Jb > 0.0 ? Jb : 0.0) * hbl;
                 const double w = p.gustiness_parameter * (x < 1e-30 ? 0.0 : ne_cbrt_ge1(x));
