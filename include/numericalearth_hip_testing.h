@@ -55,6 +55,12 @@ int ne_exp_f64(ne_ctx* ctx, const double* x, double* y, int64_t n, void* stream)
 int ne_stream_probe_f64(ne_ctx* ctx, const double* const* in, int32_t n_in, double* const* out, int32_t n_out,
                         int64_t n, void* stream);
 
+/* How the tracer stage and tendency kernels of a single model cut an Nx × Ny × Nz grid on a device of
+ * `compute_units`, each of which holds `waves` of their blocks: out[0] tiles of 63×4 columns, of which the
+ * first out[1] are taken in chunks of out[2] levels and the others in chunks of out[3]. Computed on the
+ * host; needs no device. */
+int ne_stage_plan(int32_t Nx, int32_t Ny, int32_t Nz, int32_t waves, int32_t compute_units, int32_t out[4]);
+
 #ifdef __cplusplus
 }
 #endif

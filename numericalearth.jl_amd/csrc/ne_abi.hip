@@ -242,7 +242,7 @@ size_t freeze_flag_bytes(const ne_model_desc& d) {
 
 // The model's rounding residual (totals and tile partials), rounded up to 256 bytes.
 size_t residual_bytes(const ne_model_desc& d) {
-    return ((size_t)residual_slots(grid_dev(d.grid)) * RESIDUAL_SLOT * sizeof(double) + 255) & ~(size_t)255;
+    return ((size_t)residual_capacity(grid_dev(d.grid)) * RESIDUAL_SLOT * sizeof(double) + 255) & ~(size_t)255;
 }
 
 // The deferred-column list of the FP32 flux solve: a count and one int per column, rounded up to
@@ -339,6 +339,11 @@ int ne_ctx_create(int device, ne_ctx** out) {
     ne_ctx* c = new (std::nothrow) ne_ctx();
     if (!c) return NE_ERR_CAPACITY;
     c->device = device;
+    if (hipDeviceGetAttribute(&c->compute_units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        c->compute_units <= 0) {
+        delete c;
+        return NE_ERR_DEVICE;
+    }
     c->scratch = nullptr;
     c->scratch_bytes = 0;
     if (hipMalloc((void**)&c->counters, COUNTER_BYTES) != hipSuccess) { delete c; return NE_ERR_DEVICE; }
@@ -455,6 +460,21 @@ int ne_stream_probe_f64(ne_ctx* c, const double* const* in, int32_t n_in, double
     return dev_err(launch_stream_probe(in, n_in, out, n_out, n, as_stream(stream)));
 }
 
+int ne_stage_plan(int32_t Nx, int32_t Ny, int32_t Nz, int32_t waves, int32_t compute_units, int32_t out[4]) {
+    if (!out) return NE_ERR_NULL;
+    if (Nx <= 0 || Ny <= 0 || Nz <= 0 || Nz > NE_MAX_LEVELS || waves <= 0 || compute_units <= 0) return NE_ERR_SHAPE;
+    GridDev g = {};
+    g.Nx = Nx;
+    g.Ny = Ny;
+    g.Nz = Nz;
+    const StagePlan p = stage_plan(g, waves, compute_units);
+    out[0] = p.tiles;
+    out[1] = p.first;
+    out[2] = p.levels;
+    out[3] = p.rest_levels;
+    return NE_OK;
+}
+
 int ne_fractional_indices_nodes_f64(ne_ctx* c, const ne_grid* g, const double* lambda_nodes, int32_t nx,
                                     int32_t topology_x, const double* phi_nodes, int32_t ny, int32_t topology_y,
                                     double* fi, double* fj, void* stream) {
@@ -544,7 +564,7 @@ int ne_tracer_tendency_weno5_f64(ne_ctx* c, const ne_grid* g, const ne_params* p
                                    view<const double>(o->w), view<const double>(o->T), view<const double>(o->S),
                                    view<const double>(net->J_T), view<const double>(net->J_S),
                                    view<const double>(net->J_w), tracer_forcing(p, *net), view<double>(GT),
-                                   view<double>(GS), as_stream(stream)));
+                                   view<double>(GS), c->compute_units, as_stream(stream)));
 }
 
 int ne_tracer_ab2_update_f64(ne_ctx* c, const ne_grid* g, ne_view T, ne_view S, ne_view GT, ne_view GS,
@@ -583,7 +603,8 @@ int ne_tracer_rk_stage_f64(ne_ctx* c, const ne_grid* g, const ne_params* p, ne_v
                                            view<const double>(Tin), view<const double>(Sin), view<double>(Tout),
                                            view<double>(Sout), view<const double>(net->J_T),
                                            view<const double>(net->J_S), view<const double>(net->J_w),
-                                           tracer_forcing(p, *net), beta_dt, false, 0.0, as_stream(stream)));
+                                           tracer_forcing(p, *net), beta_dt, false, 0.0, c->compute_units,
+                                           as_stream(stream)));
 }
 
 // FP32 forms of the per-phase entry points (the mixed form's convention): FP32 prescribed series
@@ -621,7 +642,7 @@ int ne_tracer_tendency_weno5_f32(ne_ctx* c, const ne_grid* g, const ne_params* p
                                           view<const float>(o->w), view<const float>(o->T), view<const float>(o->S),
                                           view<const double>(net->J_T), view<const double>(net->J_S),
                                           view<const double>(net->J_w), tracer_forcing(p, *net), view<float>(GT),
-                                          view<float>(GS), as_stream(stream)));
+                                          view<float>(GS), c->compute_units, as_stream(stream)));
 }
 
 int ne_tracer_rk_stage_f32(ne_ctx* c, const ne_grid* g, const ne_params* p, ne_view u, ne_view v, ne_view w,
@@ -641,7 +662,8 @@ int ne_tracer_rk_stage_f32(ne_ctx* c, const ne_grid* g, const ne_params* p, ne_v
                                           view<const float>(Tin), view<const float>(Sin), view<float>(Tout),
                                           view<float>(Sout), view<const double>(net->J_T),
                                           view<const double>(net->J_S), view<const double>(net->J_w),
-                                          tracer_forcing(p, *net), beta_dt, false, 0.0, as_stream(stream)));
+                                          tracer_forcing(p, *net), beta_dt, false, 0.0, c->compute_units,
+                                           as_stream(stream)));
 }
 
 int ne_compute_w_from_continuity_f64(ne_ctx* c, const ne_grid* g, ne_view u, ne_view v, ne_view w, void* stream) {
@@ -759,7 +781,7 @@ static int model_ab2_step(ne_model* m, double dt, hipStream_t s, hipEvent_t* ev)
                                            view<const double>(d.ocean.w), view<const double>(d.ocean.T),
                                            view<const double>(d.ocean.S), view<const double>(d.net.J_T),
                                            view<const double>(d.net.J_S), view<const double>(d.net.J_w), F,
-                                           view<double>(GT), view<double>(GS), s);
+                                           view<double>(GT), view<double>(GS), m->ctx->compute_units, s);
     if (e != hipSuccess) return NE_ERR_DEVICE;
     if (ev && hipEventRecord(ev[1], s) != hipSuccess) return NE_ERR_DEVICE;
     e = launch_ab2_update(g, view<double>(d.ocean.T), view<double>(d.ocean.S), view<const double>(GT),
@@ -781,18 +803,19 @@ static int model_ocean_step(ne_model* m, double dt, hipStream_t s, hipEvent_t* e
     View3<const double> JT = view<const double>(d.net.J_T), JS = view<const double>(d.net.J_S),
                         Jw = view<const double>(d.net.J_w);
     const double beta[3] = {1.0 / 3.0, 0.5, 1.0};
+    const int cus = m->ctx->compute_units;
     hipError_t e;
     if (ev && hipEventRecord(ev[0], s) != hipSuccess) return NE_ERR_DEVICE;
     const bool sr = sizeof(Real) == 4;   // FP32 state: stochastic rounding of the stage that writes it
     TracerForcing F = tracer_forcing(&d.params, d.net);
     if (F.two_color) F.beer = m->beer;   // the factors filled at creation
     e = launch_rk_stage<Real>(g, u, v, w, T0, S0, T0, S0, view<Real>(m->vT1), view<Real>(m->vS1), JT, JS, Jw, F,
-                              beta[0] * dt, false, m->time, s);
+                              beta[0] * dt, false, m->time, cus, s);
     if (e != hipSuccess) return NE_ERR_DEVICE;
     if (ev && hipEventRecord(ev[1], s) != hipSuccess) return NE_ERR_DEVICE;
     e = launch_rk_stage<Real>(g, u, v, w, T0, S0, view<const Real>(m->vT1), view<const Real>(m->vS1),
                               view<Real>(m->vT2), view<Real>(m->vS2), JT, JS, Jw, F, beta[1] * dt, false, m->time,
-                              s);
+                              cus, s);
     if (e != hipSuccess) return NE_ERR_DEVICE;
     if (ev && hipEventRecord(ev[2], s) != hipSuccess) return NE_ERR_DEVICE;
     TracerForcing F3 = F;   // the last stage flags the columns the freeze clamp visits
@@ -802,7 +825,7 @@ static int model_ocean_step(ne_model* m, double dt, hipStream_t s, hipEvent_t* e
     if (sr) F3.residual = m->residual;   // and an FP32 state's rounding residual
     e = launch_rk_stage<Real>(g, u, v, w, T0, S0, view<const Real>(m->vT2), view<const Real>(m->vS2),
                               view<Real>(d.ocean.T), view<Real>(d.ocean.S), JT, JS, Jw, F3, beta[2] * dt, sr, m->time,
-                              s);
+                              cus, s);
     if (e != hipSuccess) return NE_ERR_DEVICE;
     if (ev && hipEventRecord(ev[3], s) != hipSuccess) return NE_ERR_DEVICE;
     return NE_OK;
@@ -1059,7 +1082,8 @@ int ne_model_snapshot_resident(ne_model* m, int32_t which, int64_t position) {
 
 int ne_model_rounding_residual(const ne_model* m, double* out, void* stream) {
     if (!m || !out) return NE_ERR_NULL;
-    return dev_err(launch_residual_reduce(m->residual, grid_dev(m->d.grid), out, as_stream(stream)));
+    return dev_err(launch_residual_reduce(m->residual, grid_dev(m->d.grid), m->ctx->compute_units, out,
+                                          as_stream(stream)));
 }
 
 int ne_model_clock(const ne_model* m, double* time, int64_t* iteration) {

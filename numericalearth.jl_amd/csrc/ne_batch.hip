@@ -29,7 +29,6 @@ using namespace ne;
 
 namespace {
 
-constexpr int NXCD = 8;
 constexpr int TILE_ROWS[3] = {4, 8, 16};
 constexpr int SURFACE_BLOCKS[3] = {64, 128, 256};
 
@@ -82,7 +81,6 @@ struct ne_batch {
     bool unit = false;   // every member's fields have the unit layouts
 
     ne_batch_tuning tuning;
-    int cus = 256;
     bool use_graph = false;
     hipStream_t capture_stream = nullptr;
     hipGraph_t graph = nullptr;
@@ -177,7 +175,7 @@ BatchRec<Real> member_record(const ne_model* m, const double* atimes_dev, const 
     r.freeze_flags = m->freeze_flags;
     r.residual = m->residual;
     r.beer = m->beer;
-    r.levels = stage_levels(r.g, tile_levels);
+    r.levels = stage_levels(r.g, tile_levels, m->ctx->compute_units);
     r.atimes = atimes_dev;
     r.rtimes = rtimes_dev;
     r.nat = (int)m->atimes.size();
@@ -208,7 +206,7 @@ int rebuild(ne_batch* b, hipStream_t s) {
         const ne_model* m = b->members[k];
         const ne_grid& g = m->d.grid;
         const int tc = m->d.params.radiative_forcing == NE_RADIATIVE_FORCING_TWO_COLOR ? 1 : 0;
-        const int chunks = level_chunks(g.Nz, stage_levels(grid_dev(g), tile_levels));
+        const int chunks = level_chunks(g.Nz, stage_levels(grid_dev(g), tile_levels, m->ctx->compute_units));
         for (int c = 0; c < 3; c++) {
             int nt = batch_tiles_x(g.Nx) * batch_tiles_y(g.Ny, TILE_ROWS[c]) * chunks;
             for (int t = 0; t < nt; t++) {
@@ -380,7 +378,7 @@ int autotune(ne_batch* b, hipStream_t s, ne_batch_tuning* out) {
         if (nwork == 0) continue;
         const int per_cu[4] = {1, 2, 4, 0};
         for (int pc : per_cu) {
-            const int blocks = pc ? std::max(NXCD, std::min(round8(nwork), pc * b->cus)) : round8(nwork);
+            const int blocks = pc ? std::max(NXCD, std::min(round8(nwork), pc * b->ctx->compute_units)) : round8(nwork);
             double ms;
             auto f = [&]() {
                 // both forcing lists, each with the grid the step would give it
@@ -410,7 +408,7 @@ int autotune(ne_batch* b, hipStream_t s, ne_batch_tuning* out) {
         if (b->surface_nwork[c] == 0) continue;
         const int per_cu[4] = {2, 4, 8, 0};
         for (int pc : per_cu) {
-            int req = pc ? pc * b->cus : 0;
+            int req = pc ? pc * b->ctx->compute_units : 0;
             double ms;
             auto f = [&]() {
                 hipError_t e = hipSuccess;
@@ -480,9 +478,6 @@ int ne_batch_create(ne_ctx* c, int32_t precision, int n, ne_model* const* models
         }
         b->members.push_back(models[k]);
     }
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess && cus > 0)
-        b->cus = cus;
     default_tuning(b);
     int r = NE_OK;
     for (int i = 0; i < 2 && !r; i++)

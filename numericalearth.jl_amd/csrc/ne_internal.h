@@ -14,6 +14,7 @@ static_assert(sizeof(ne_counters) <= COUNTER_STRIPE_BYTES, "a stripe holds the c
 
 struct ne_ctx {
     int device;
+    int compute_units;
     ne_counters* counters;      // device, COUNTER_STRIPES copies of COUNTER_STRIPE_BYTES each
     double* scratch;            // device workspace (budget partials), grown on demand
     size_t scratch_bytes;
@@ -31,7 +32,7 @@ struct ne_model {
     // one byte per column, set by the step's last RK stage where a cell of the column is below its
     // freezing point, so the freeze clamp that follows visits only those and clears them
     uint8_t* freeze_flags = nullptr;
-    // rounding residual of the FP32 state (residual_bytes): per tile, the running compensated
+    // rounding residual of the FP32 state (residual_bytes): per tile and chunk of levels, the running compensated
     // totals Σ V·(x − stored) of T and S (sum, compensation, sum, compensation)
     double* residual = nullptr;
     // columns the FP32 flux solve leaves to its second kernel (count, then one int per column)
@@ -175,7 +176,7 @@ hipError_t launch_rk_stage(const GridDev& g, View3<const Real> u, View3<const Re
                            View3<const Real> T0, View3<const Real> S0, View3<const Real> Tin,
                            View3<const Real> Sin, View3<Real> Tout, View3<Real> Sout, View3<const double> JT,
                            View3<const double> JS, View3<const double> Jw, TracerForcing forcing, double beta_dt,
-                           bool stochastic, double time, hipStream_t s);
+                           bool stochastic, double time, int compute_units, hipStream_t s);
 
 // Seed of a step's stochastic rounding: a hash of the bits of the model time.
 __host__ __device__ inline uint32_t step_seed(double time) {
@@ -197,7 +198,7 @@ template <typename Real>
 hipError_t launch_tendency(const GridDev& g, View3<const Real> u, View3<const Real> v, View3<const Real> w,
                            View3<const Real> T, View3<const Real> S, View3<const double> JT,
                            View3<const double> JS, View3<const double> Jw, TracerForcing forcing, View3<Real> GT,
-                           View3<Real> GS, hipStream_t s);
+                           View3<Real> GS, int compute_units, hipStream_t s);
 // Quasi-Adams–Bashforth 2 update of an FP64 state from the step's tendency G and the last
 // step's G⁻ (not read when euler), with the freeze flags of the step (ne_tracer.hip).
 hipError_t launch_ab2_update(const GridDev& g, View3<double> T, View3<double> S, View3<const double> GT,
@@ -220,7 +221,8 @@ hipError_t launch_budget_noalloc(double* partial, const GridDev& g, View3<const 
                                  double* out, hipStream_t s);
 // Rounding residual of an FP32 state: one slot per tile and chunk of levels (T sum, T compensation, S sum,
 // S compensation), into which the block of the step's last stage adds the tile's Σ V·(x −
-// stored); the number of slots a model keeps, and their fixed-order sum into out[4].
+// stored); the number of slots a model keeps, those of them a device's launches use (residual_slots),
+// and their fixed-order sum into out[4].
 constexpr int RESIDUAL_SLOT = 4;
 // Beer's-law factors of the two colours at the Nz+1 faces (TracerForcing::beer), as the stage
 // kernel would compute them in place.
@@ -232,13 +234,25 @@ hipError_t launch_halo_fill(const GridDev& g, View3<Real> c, int Hx, int Hy, int
 // Traffic probe (ne_stream_probe_f64): n_in ≤ NE_STREAM_PROBE_MAX_IN arrays read, n_out written.
 hipError_t launch_stream_probe(const double* const* in, int n_in, double* const* out, int n_out, int64_t n,
                                hipStream_t s);
-int64_t residual_slots(const GridDev& g);
+int64_t residual_capacity(const GridDev& g);
+int64_t residual_slots(const GridDev& g, int compute_units);
+constexpr int NXCD = 8;   // blocks are dealt round-robin to the chip's XCDs
+// How the single-model stage and tendency kernels cut their tiles' levels on a device of that many
+// compute units, each of which holds `waves` blocks: tiles 0 … first-1 in chunks of `levels`, the others
+// in chunks of `rest_levels`.
+struct StagePlan {
+    int tiles, first, levels, rest_levels;
+    __host__ __device__ int first_per_xcd() const { return (first + NXCD - 1) / NXCD; }
+    __host__ __device__ int rest_per_xcd() const { return (tiles - first + NXCD - 1) / NXCD; }
+};
+StagePlan stage_plan(const GridDev& g, int waves, int compute_units);
 // Levels of a tile that one block of the stage and tendency kernels takes, and the number of such
 // chunks in a column of Nz levels.
 int64_t stage_tile_levels(const GridDev& g);
-int stage_levels(const GridDev& g, int64_t tile_levels);
+int stage_levels(const GridDev& g, int64_t tile_levels, int compute_units);
 __host__ __device__ inline int level_chunks(int Nz, int levels) { return (Nz + levels - 1) / levels; }
-hipError_t launch_residual_reduce(const double* residual, const GridDev& g, double* out, hipStream_t s);
+hipError_t launch_residual_reduce(const double* residual, const GridDev& g, int compute_units, double* out,
+                                  hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Batched ensemble: one device record per member model, read by persistent kernels

@@ -70,7 +70,6 @@ constexpr int stage_waves(bool two_color, bool last) {
                              : NE_STAGE_WAVES_PER_EU_F32;
 }
 constexpr int PLAIN_TR = NE_PLAIN_TR;  // cell rows per tile of the single-model kernel
-constexpr int NXCD = 8;
 constexpr int KMIN_OUTSIDE = 1 << 30;  // kmin of a column outside a bounded domain
 
 // LDS of one tile of TR rows: the T/S plane with a 3-cell halo, the x- and y-face fluxes
@@ -90,13 +89,6 @@ struct TileShared {
 __host__ __device__ inline int tiles_x(int Nx) { return (Nx + TC - 1) / TC; }
 __host__ __device__ inline int tiles_y(int Ny, int tr) { return (Ny + tr - 1) / tr; }
 
-// How the single-model kernel cuts its tiles' levels: tiles 0 … first-1 in chunks of `levels`, the
-// others in chunks of `rest_levels` (stage_plan).
-struct StagePlan {
-    int tiles, first, levels, rest_levels;
-    __host__ __device__ int first_per_xcd() const { return (first + NXCD - 1) / NXCD; }
-    __host__ __device__ int rest_per_xcd() const { return (tiles - first + NXCD - 1) / NXCD; }
-};
 inline int grid_blocks(const StagePlan& p, int Nz) {
     return NXCD * (p.first_per_xcd() * level_chunks(Nz, p.levels) + p.rest_per_xcd() * level_chunks(Nz, p.rest_levels));
 }
@@ -891,54 +883,54 @@ TracerLayout host_layout(const View3<const Real>& c, const View3<const Real>& u,
 
 // Levels of one block. A block takes its levels in series, about 2.7 µs each when the chip is not
 // full, so a grid (or batch) of few tiles has each tile's column cut into chunks until there are
-// about NE_STAGE_TARGET_BLOCKS blocks; every chunk pays the tile's set-up and one more z face
-// (≈ 1.5 levels), so full grids are not cut. 1024 blocks of the FP64 kernel are resident at once;
-// 1536 measured best over 768 … 3072 (whole steps, uncut → cut, µs: one column of 50 levels
+// about NE_STAGE_BLOCKS_PER_CU blocks for each compute unit; every chunk pays the tile's set-up and one
+// more z face (≈ 1.5 levels), so full grids are not cut. Four blocks of the FP64 kernel are resident on
+// a compute unit at once; 6, 1536 on the chip's 256, measured best over 768 … 3072 (whole steps, uncut
+// → cut, µs: one column of 50 levels
 // 166 → 57, 90×40×10 139 → 89, 353×137×19 mixed 235 → 142, 481×187×23 578 → 485, 12 uneven FP64
-// members 448 → 362 and mixed ones 295 → 122; 1440×560×10 has 3220 tiles and stays uncut: two chunks
-// per tile took its FP64 stage from 136 to 151 µs).
-#ifndef NE_STAGE_TARGET_BLOCKS
-#define NE_STAGE_TARGET_BLOCKS 1536
+// members 448 → 362 and mixed ones 295 → 122; two chunks for each of 1440×560×10's 3220 tiles took its
+// FP64 stage from 136 to 151 µs, so there only the tiles left over from full rounds are cut: stage_plan).
+#ifndef NE_STAGE_BLOCKS_PER_CU
+#define NE_STAGE_BLOCKS_PER_CU 6
 #endif
+constexpr int CHIP_CUS = 256;   // of an MI355X; a partition of it has fewer (residual_capacity)
 int64_t stage_tile_levels(const GridDev& g) { return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR) * g.Nz; }
 
-int stage_levels(const GridDev& g, int64_t tile_levels) {
-    const int64_t wanted = std::max<int64_t>((tile_levels + NE_STAGE_TARGET_BLOCKS - 1) / NE_STAGE_TARGET_BLOCKS, 1);
+int stage_levels(const GridDev& g, int64_t tile_levels, int compute_units) {
+    const int64_t target = NE_STAGE_BLOCKS_PER_CU * std::min(compute_units, CHIP_CUS);
+    const int64_t wanted = std::max<int64_t>((tile_levels + target - 1) / target, 1);
     const int chunks = (int)((g.Nz + wanted - 1) / wanted);
     return (g.Nz + chunks - 1) / chunks;
 }
 
-namespace {
 // The chip holds `waves` 4-wavefront blocks of a stage kernel per CU at once. A launch of more tiles
 // than that ends with a partly filled round of whole columns, so the tiles left over from full rounds
 // are cut into as many chunks as have a place in one (each chunk costs a set-up of about 1½ levels,
-// which the idle places pay). 1440×560×10 has 3220 tiles: 148 are left over from 3 rounds of 1024
+// which the idle places pay). On 256 CUs 1440×560×10 has 3220 tiles: 148 are left over from 3 rounds of 1024
 // (FP64), or from 2 of 1536 (the mixed form's last stage), and the stages took 128 against 132 µs and
 // 91 against 93; from 1 of 1792 (its other stages) 1428 are, more than half a round, and stay whole.
 // Cutting 256 or 1024 tiles more took the FP64 stage to 130 and 134 µs. Grids of fewer tiles than
 // places are cut throughout (stage_levels).
-constexpr int CUS = 256;
-StagePlan stage_plan(const GridDev& g, int waves) {
-    const int tiles = tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR), places = waves * CUS;
+StagePlan stage_plan(const GridDev& g, int waves, int compute_units) {
+    const int tiles = tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR), places = waves * compute_units;
     if (tiles < places) {
-        const int levels = stage_levels(g, stage_tile_levels(g));
+        const int levels = stage_levels(g, stage_tile_levels(g), compute_units);
         return {tiles, tiles, levels, levels};
     }
     const int rest = tiles % places;
     const int chunks = rest > 0 ? std::min(places / rest, g.Nz) : 1;
     return {tiles, chunks > 1 ? tiles - rest : tiles, g.Nz, (g.Nz + chunks - 1) / chunks};
 }
-}  // namespace
 
 template <typename Real>
 hipError_t launch_rk_stage(const GridDev& g, View3<const Real> u, View3<const Real> v, View3<const Real> w,
                            View3<const Real> T0, View3<const Real> S0, View3<const Real> Tin, View3<const Real> Sin,
                            View3<Real> Tout, View3<Real> Sout, View3<const double> JT, View3<const double> JS,
                            View3<const double> Jw, TracerForcing forcing, double beta_dt, bool stochastic,
-                           double time, hipStream_t s) {
+                           double time, int compute_units, hipStream_t s) {
     TracerLayout L = host_layout<Real>(Tin, u, v, w, JT);
     const bool watch = forcing.freeze_flags != nullptr;
-    const StagePlan plan = stage_plan(g, stage_waves<Real>(forcing.two_color != 0, watch));
+    const StagePlan plan = stage_plan(g, stage_waves<Real>(forcing.two_color != 0, watch), compute_units);
     const dim3 grid(grid_blocks(plan, g.Nz)), block(TW, PLAIN_TR);
     const int sr = stochastic ? 1 : 0;
     const uint32_t seed = step_seed(time);
@@ -973,12 +965,12 @@ template hipError_t launch_rk_stage<double>(const GridDev&, View3<const double>,
                                             View3<const double>, View3<const double>, View3<const double>,
                                             View3<const double>, View3<const double>, View3<double>, View3<double>,
                                             View3<const double>, View3<const double>, View3<const double>,
-                                            TracerForcing, double, bool, double, hipStream_t);
+                                            TracerForcing, double, bool, double, int, hipStream_t);
 template hipError_t launch_rk_stage<float>(const GridDev&, View3<const float>, View3<const float>,
                                            View3<const float>, View3<const float>, View3<const float>,
                                            View3<const float>, View3<const float>, View3<float>, View3<float>,
                                            View3<const double>, View3<const double>, View3<const double>,
-                                           TracerForcing, double, bool, double, hipStream_t);
+                                           TracerForcing, double, bool, double, int, hipStream_t);
 
 // Quasi-Adams–Bashforth 2 update (the reference's timestepper = :QuasiAdamsBashforth2,
 // ocean_simulation.jl:323, with Oceananigans' default χ = 0.1): in every active cell
@@ -1021,9 +1013,9 @@ template <typename Real>
 hipError_t launch_tendency(const GridDev& g, View3<const Real> u, View3<const Real> v, View3<const Real> w,
                            View3<const Real> T, View3<const Real> S, View3<const double> JT,
                            View3<const double> JS, View3<const double> Jw, TracerForcing forcing, View3<Real> GT,
-                           View3<Real> GS, hipStream_t s) {
+                           View3<Real> GS, int compute_units, hipStream_t s) {
     TracerLayout L = host_layout<Real>(T, u, v, w, JT);
-    const StagePlan plan = stage_plan(g, stage_waves<Real>(forcing.two_color != 0, false));
+    const StagePlan plan = stage_plan(g, stage_waves<Real>(forcing.two_color != 0, false), compute_units);
     const dim3 grid(grid_blocks(plan, g.Nz)), block(TW, PLAIN_TR);
     if (forcing.two_color)
         hipLaunchKernelGGL((tracer_tile_kernel<Real, 1, true>), grid, block, 0, s, g, L, u.p, v.p, w.p, T.p, S.p, T.p,
@@ -1036,11 +1028,11 @@ hipError_t launch_tendency(const GridDev& g, View3<const Real> u, View3<const Re
 template hipError_t launch_tendency<double>(const GridDev&, View3<const double>, View3<const double>,
                                             View3<const double>, View3<const double>, View3<const double>,
                                             View3<const double>, View3<const double>, View3<const double>,
-                                            TracerForcing, View3<double>, View3<double>, hipStream_t);
+                                            TracerForcing, View3<double>, View3<double>, int, hipStream_t);
 template hipError_t launch_tendency<float>(const GridDev&, View3<const float>, View3<const float>,
                                            View3<const float>, View3<const float>, View3<const float>,
                                            View3<const double>, View3<const double>, View3<const double>,
-                                           TracerForcing, View3<float>, View3<float>, hipStream_t);
+                                           TracerForcing, View3<float>, View3<float>, int, hipStream_t);
 
 template <typename Real>
 hipError_t launch_budget(ne_ctx* ctx, const GridDev& g, View3<const Real> c, double weight, double* out,
@@ -1100,19 +1092,29 @@ int64_t budget_blocks(const GridDev& g) {
 // One slot of 4 doubles per block of the FP32 state's last stage: the single-model kernel's, or the
 // batch's of its 4-row tiles with no shorter chunks than the grid alone would have (taller tiles use
 // the first slots).
-int64_t residual_slots(const GridDev& g) {
+int64_t residual_slots(const GridDev& g, int compute_units) {
     int64_t n = (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR < 4 ? PLAIN_TR : 4) *
-                level_chunks(g.Nz, stage_levels(g, stage_tile_levels(g)));
+                level_chunks(g.Nz, stage_levels(g, stage_tile_levels(g), compute_units));
     for (bool two_color : {false, true}) {
-        const StagePlan p = stage_plan(g, stage_waves<float>(two_color, true));
+        const StagePlan p = stage_plan(g, stage_waves<float>(two_color, true), compute_units);
         n = std::max<int64_t>(n, (int64_t)p.first * level_chunks(g.Nz, p.levels) +
                                      (int64_t)(p.tiles - p.first) * level_chunks(g.Nz, p.rest_levels));
     }
     return n;
 }
 
-hipError_t launch_residual_reduce(const double* residual, const GridDev& g, double* out, hipStream_t s) {
-    hipLaunchKernelGGL(residual_reduce_kernel, dim3(1), dim3(RB), 0, s, residual, (int)residual_slots(g), out);
+// At least residual_slots of any number of compute units, for a workspace that is sized before its
+// device is known: fewer compute units than a chip's ask for fewer chunks, and the tiles left over from
+// full rounds take at most one round's places, no more than there are tiles.
+int64_t residual_capacity(const GridDev& g) {
+    return (int64_t)tiles_x(g.Nx) * tiles_y(g.Ny, PLAIN_TR < 4 ? PLAIN_TR : 4) *
+           std::max(level_chunks(g.Nz, stage_levels(g, stage_tile_levels(g), CHIP_CUS)), std::min(g.Nz, 2));
+}
+
+hipError_t launch_residual_reduce(const double* residual, const GridDev& g, int compute_units, double* out,
+                                  hipStream_t s) {
+    hipLaunchKernelGGL(residual_reduce_kernel, dim3(1), dim3(RB), 0, s, residual, (int)residual_slots(g, compute_units),
+                       out);
     return hipGetLastError();
 }
 

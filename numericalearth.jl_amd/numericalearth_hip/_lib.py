@@ -43,6 +43,7 @@ SIGNATURES = {
     "ne_sqrt_f64": [vp, vp, vp, C.c_int64, vp],
     "ne_exp_f64": [vp, vp, vp, C.c_int64, vp],
     "ne_stream_probe_f64": [vp, vp, C.c_int32, vp, C.c_int32, C.c_int64, vp],
+    "ne_stage_plan": [C.c_int32] * 5 + [P(C.c_int32)],
     "ne_fill_halo_f64": [vp, vp, abi.View, C.c_int32, C.c_int32, C.c_int32, vp],
     "ne_fill_halo_f32": [vp, vp, abi.View, C.c_int32, C.c_int32, C.c_int32, vp],
     "ne_fractional_indices_nodes_f64": [vp, P(abi.Grid), vp, C.c_int32, C.c_int32, vp, C.c_int32, C.c_int32, vp, vp,
