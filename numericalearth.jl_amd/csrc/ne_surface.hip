@@ -22,6 +22,13 @@ constexpr int BY = 4;
 #ifndef NE_FLUX_WAVES_PER_EU
 #define NE_FLUX_WAVES_PER_EU 4
 #endif
+// The general path's iteration needs more than 4 wavefronts leave it: with 128 registers it spills 177 to 211
+// of them around the library's functions, and how long an iteration takes depends on where (the shared
+// offsets made the COARE profile of the mixed form 4 % slower and of FP64 5 % faster). With 256 it
+// spills 18 to 30 (the batch's 241): update of 1440×560, µs with 4, 3 and 2 wavefronts, FP64: COARE 2136, 1804,
+// 1089; skin temperature 4838, 4430, 2785; no stability functions 879, 702, 464; mixed 2368, 1782, 1076;
+// 4799, 4384, 2750; 947, 678, 442; COARE at 90×40 644, 497, 316 and 711, 500, 315.
+constexpr int flux_waves(int path) { return path == 0 ? 2 : NE_FLUX_WAVES_PER_EU; }
 
 // 1: the mixed form (FP32 storage) starts the fixed point with the FP32 pre-iteration;
 // 0: it runs the FP64 iteration of the FP64 form from the reference's initial guess.
@@ -369,7 +376,7 @@ __device__ __forceinline__ void ocean_surface(const GridDev& g, const View3<cons
 }
 
 template <int PATH, bool UNIT>
-__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
+__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(flux_waves(PATH))))
 flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3<const double> va,
                                            View3<const double> Ta, View3<const double> pa, View3<const double> qa,
                                            View3<const double> T, View3<const double> S, View3<const double> u,
@@ -414,7 +421,7 @@ flux_solve_exchange_kernel(GridDev g, ne_params p, View3<const double> ua, View3
 // beyond a bounded edge is inactive (zero interface state). The solve runs as in the interior
 // (same instance of the column solve); the ring is not counted in the solver counters.
 template <int PATH>
-__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
+__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(flux_waves(PATH))))
 flux_solve_ring_kernel(GridDev g, ne_params p, View3<const double> ua, View3<const double> va,
                        View3<const double> Ta, View3<const double> pa, View3<const double> qa,
                        View3<const double> T, View3<const double> S, View3<const double> u,
@@ -680,7 +687,7 @@ __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const 
 // iteration does not finish it is appended to `deferred` (count, then flattened columns) and left
 // to surface_deferred_kernel.
 template <typename Real, int PATH, bool UNIT, bool Defer = false>
-__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
+__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(flux_waves(PATH))))
 surface_update_kernel(GridDev g, ne_params p, AtmosDev<Real> a, const double* __restrict__ fi,
                       const double* __restrict__ fj, RadDev<Real> rd, const double* __restrict__ rfi,
                       const double* __restrict__ rfj, View3<Real> T, View3<const Real> S, View3<const Real> u,
@@ -787,7 +794,7 @@ __global__ void __launch_bounds__(BX* BY) surface_tau_kernel(GridDev g, ne_param
 // flagged columns, net fluxes other than τ, radiation); without it (the autotuner's timing
 // runs) the kernel only solves, leaving the state as it is.
 template <typename Real, int PATH, bool UNIT, bool FUSED>
-__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(NE_FLUX_WAVES_PER_EU)))
+__global__ void __launch_bounds__(BX* BY) __attribute__((amdgpu_waves_per_eu(flux_waves(PATH))))
 batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem* __restrict__ work, int nwork,
                            double dt_frazil, ne_counters* counters) {
     __shared__ FluxTable<Real, PATH> tab;
