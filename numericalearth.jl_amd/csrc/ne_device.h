@@ -1423,14 +1423,17 @@ __host__ __device__ inline ne_time_interp time_indices(const double* times, int 
 // The face value is c₂ + Σ_r ω_r (q_r − c₂): a uniform field gives c₂ exactly, and the
 // reconstruction of the mirrored values is the negated reconstruction of the negated
 // differences, so the upwind side is chosen by selecting differences. Scaling every β_r
-// and ε by the same factor leaves the weights unchanged: 4β_r + 4ε = (13/3)s_r² + e_r² + 4ε is two
-// fused operations. With the linear weights as 1 : 6 : 3 and 6(q_r − c₂) = 2e₀ − δ₁, e₁ + δ₂, e₂ + δ₂
+// and ε by the same factor leaves the weights unchanged: 4β_r + 4ε = (13/3)s_r² + e_r² + 4ε (FP64) or
+// 12/13 (β_r + ε) (FP32) is two fused operations. With the linear weights as 1 : 6 : 3 and 6(q_r − c₂) = 2e₀ − δ₁, e₁ + δ₂, e₂ + δ₂
 // the cores return Σ α_r 6(q_r − c₂) / Σ α_r, and the 1/6 joins the sign of the flow in the one
 // fused operation that adds it to c₂. The FP64 weights are normalised with one division:
 // multiplying every α_r = d_r (1 + (τ/(β_r+ε))²) by Π_s (β_s+ε)² leaves α_r/Σα unchanged;
 // the division is a reciprocal refined by two Newton steps (within 2 ulp). In FP32 the
 // Π(β+ε)² products could underflow, so FP32 forms the three 1/(β_r+ε) from one reciprocal of
-// Π(β+ε) (at least (4ε)³) and the other two factors, and normalises with a second.
+// Π(β+ε) and the other two factors, and normalises with a second. That product and the squares of
+// the weights bound FP32's range, so its factor is 12/13 and not 4 (64 times the product) and its linear
+// weights are an eighth of 1 : 6 : 3: WENO5 holds for differences of neighbours up to 7·10⁵, and steps
+// between constant values up to 2.3·10⁵ (with the FP64 form's factors 3.6·10⁵ and 1.5·10⁵).
 // Fused multiply-adds are allowed here (contract(fast)). With ε added apart, weights of 0.1, 0.6, 0.3 and
 // the 1/6 in the denominator (about 8 operations of 70 a face more) the stages of 1440×560×10 took 136 µs
 // (FP64) and 82 (mixed) against 130 and 75.
@@ -1456,22 +1459,21 @@ __device__ __forceinline__ double weno5z_core(double d0, double d1, double d2, d
 
 __device__ __forceinline__ float weno5z_core(float d0, float d1, float d2, float d3) {
 #pragma clang fp contract(fast)
-    const float eps4 = 4.0f * (float)NE_WENO_EPS;
-    const float k = 2.081666f;   // √(13/3)
-    const float s0 = k * (d1 - d0), s1 = k * (d2 - d1), s2 = k * (d3 - d2);
+    const float eps = (float)(12.0 / 13.0 * NE_WENO_EPS), c = (float)(3.0 / 13.0);   // 12/13 of β_r + ε
+    const float s0 = d1 - d0, s1 = d2 - d1, s2 = d3 - d2;
     const float e0 = fmaf(3.0f, d1, -d0), e1 = d1 + d2, e2 = fmaf(3.0f, d2, -d3);
-    const float b0 = fmaf(s0, s0, fmaf(e0, e0, eps4));
-    const float b1 = fmaf(s1, s1, fmaf(e1, e1, eps4));
-    const float b2 = fmaf(s2, s2, fmaf(e2, e2, eps4));
+    const float b0 = fmaf(s0, s0, fmaf(c * e0, e0, eps));
+    const float b1 = fmaf(s1, s1, fmaf(c * e1, e1, eps));
+    const float b2 = fmaf(s2, s2, fmaf(c * e2, e2, eps));
     // 1/(βᵣ+ε) from one reciprocal of the product and the other two factors
     const float b12 = b1 * b2;
     const float tq = (b0 - b2) * __builtin_amdgcn_rcpf(b0 * b12);   // τ's sign leaves the squares
     const float g0 = tq * b12;
     const float g1 = tq * (b0 * b2);
     const float g2 = tq * (b0 * b1);
-    const float a0 = fmaf(g0, g0, 1.0f);
-    const float a1 = 6.0f * fmaf(g1, g1, 1.0f);
-    const float a2 = 3.0f * fmaf(g2, g2, 1.0f);
+    const float a0 = 0.125f * fmaf(g0, g0, 1.0f);
+    const float a1 = 0.75f * fmaf(g1, g1, 1.0f);
+    const float a2 = 0.375f * fmaf(g2, g2, 1.0f);
     return fmaf(a0, fmaf(2.0f, e0, -d1), fmaf(a1, e1 + d2, a2 * (e2 + d2))) * __builtin_amdgcn_rcpf(a0 + a1 + a2);
 }
 
@@ -1494,8 +1496,8 @@ __device__ __forceinline__ float weno3z_core(float d0, float d1) {
     const float tau = b0 - b1;
     const float g0 = tau * __builtin_amdgcn_rcpf(b0);
     const float g1 = tau * __builtin_amdgcn_rcpf(b1);
-    const float a0 = fmaf(g0, g0, 1.0f);
-    const float a1 = 2.0f * fmaf(g1, g1, 1.0f);
+    const float a0 = 0.5f * fmaf(g0, g0, 1.0f);
+    const float a1 = fmaf(g1, g1, 1.0f);
     return fmaf(a0, d0, a1 * d1) * __builtin_amdgcn_rcpf(a0 + a1);
 }
 
