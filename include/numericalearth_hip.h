@@ -487,7 +487,8 @@ int ne_compute_w_from_continuity_f64(ne_ctx* ctx, const ne_grid* grid, ne_view u
                                      void* stream);
 
 /* Compensated (Neumaier, double-double combine) sum over active cells of
- * weight·V·c, V = Az·Δz. Writes {sum, compensation} (2 doubles) to device `out`. */
+ * weight·V·c, V = Az·Δz. Writes {sum, compensation} (2 doubles) to `out`, device memory or
+ * pinned host memory, which the caller reads after waiting for the stream. */
 int ne_budget_f64(ne_ctx* ctx, const ne_grid* grid, ne_view c, double weight,
                   double* out, void* stream);
 int ne_budget_f32(ne_ctx* ctx, const ne_grid* grid, ne_view c, double weight,

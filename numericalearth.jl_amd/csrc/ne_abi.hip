@@ -728,7 +728,7 @@ int ne_budget_f64_noalloc(ne_ctx* c, const ne_grid* g, ne_view cv, double weight
 // Model
 // ---------------------------------------------------------------------------
 
-// ev (optional): ev[3] is recorded before K1 by the caller, ev[4] after K1 and ev[5] after K2.
+// ev (optional): ev[3] is recorded before K1 by the caller, ev[4] after K1 and ev[5] after the τ kernel.
 // after_step: the state was written by the last RK stage, whose freeze flags name the columns
 // the freeze clamp has to visit; otherwise (construction, a caller's update_state) every column.
 static int model_update_state(ne_model* m, double dt_frazil, hipStream_t s, hipEvent_t* ev = nullptr,

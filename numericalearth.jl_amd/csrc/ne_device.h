@@ -308,7 +308,7 @@ __device__ __forceinline__ double psi_scalar(const ne_params& p, double z) {
 #include "ne_psi_table.h"
 #define NE_PSI_SERIES_RADIUS 5e-4
 
-// Elementary functions by precision: FP64 uses the math library (the Fast flux instance its
+// Elementary functions by precision: FP64 uses the math library (the flux paths 1 to 3 their
 // own ne_log above, ne_atan_ge1 and ne_cbrt_ge1 below); the FP32 pre-iteration of the mixed form
 // uses the hardware log₂/exp₂-based approximations.
 
@@ -987,31 +987,20 @@ __device__ __forceinline__ int flux_iterate_coefficients(const ne_params& p, dou
 // iterate_interface_fluxes(::SimilarityTheoryFluxes) (similarity:315-385).
 // Quantities that the reference re-evaluates each iteration from unchanged inputs
 // (qₛ, θᵃ, Δθ, Δq, 𝒯ₛ) are evaluated once: the values are identical.
-// Fast = true (only for the default Edson constants, edson_default_constants) evaluates the
-// two profiles with the shared/series stability functions above and R★^b as exp(b log R★).
+// PATH is the flux path (flux_path). Paths 1 to 3 (the default Edson constants,
+// edson_default_constants: Fast) evaluate the two profiles with the table and series of the stability
+// functions above and R★^b as exp(b log R★), 2 and 3 in logarithms.
 // Mixed = true (the FP32 form) runs the same fixed point in FP32 with the hardware log/exp
 // until its drift falls below NE_MIXED_DRIFT (a few times the FP32 rounding noise of
 // u★ + θ★ + q★) and takes that iterate; only a column whose FP32 iteration does not get there
 // within NE_MIXED_MAXITER iterations (or leaves the finite range) continues in FP64 from it
 // with the reference's stop criterion. Defer = true (for kernels whose parameters take the FP32
 // iteration) returns such a column as `deferred` instead of continuing: its FP64 iteration needs
-// twice the registers of the FP32 one, so the kernel that defers runs at 6 wavefronts per SIMD
-// instead of 4 and a second kernel finishes the few deferred columns with Defer = false, which
-// gives them the same values. Finishing in FP64 as well (≈ 3 more FP64 iterations)
+// half as many registers again as the FP32 one (95 to 128 against 65 to 72), so the kernel that defers
+// runs at 7 wavefronts per SIMD instead of 4 or 5 and a second kernel finishes the few deferred columns
+// with Defer = false, which gives them the same values. Finishing in FP64 as well (≈ 3 more FP64 iterations)
 // changed neither the 200-step SST error against the FP64 model (9.8e-6 of the largest SST)
 // nor the flux errors (2.4e-5 of their scale) at 1440×560×10, and cost 13 % of the step.
-// Latent heat, sensible heat and water vapour fluxes from the scales; returns the air density.
-__device__ __forceinline__ double scalar_fluxes(const ne_params& p, double Ta, double pa, double qa, double us,
-                                                double ts, double qs, double& Qv, double& Qt, double& Jv) {
-    const double rho = air_density(p, Ta, pa, qa);
-    const double cpm = cp_m(p, qa);
-    const double Lv = latent_heat_vapor(p, Ta);
-    Qv = -rho * Lv * us * qs;
-    Qt = -rho * cpm * us * ts;
-    Jv = -rho * us * qs;
-    return rho;
-}
-
 #ifndef NE_MIXED_DRIFT
 #define NE_MIXED_DRIFT 2e-7f
 #endif
@@ -1245,7 +1234,12 @@ __device__ __forceinline__ ColumnFluxes flux_column(const Tab& tab, const ne_par
     double taux = dU == 0.0 ? 0.0 : -(us * us) * du / dU;
     double tauy = dU == 0.0 ? 0.0 : -(us * us) * dv / dU;
     ColumnFluxes r;
-    const double rho = scalar_fluxes(p, Ta, pa, qa, us, ts, qs, r.Qv, r.Qt, r.Jv);
+    const double rho = air_density(p, Ta, pa, qa);
+    const double cpm = cp_m(p, qa);
+    const double Lv = latent_heat_vapor(p, Ta);
+    r.Qv = -rho * Lv * us * qs;
+    r.Qt = -rho * cpm * us * ts;
+    r.Jv = -rho * us * qs;
     r.rtx = rho * taux;
     r.rty = rho * tauy;
     r.us = us;

@@ -279,8 +279,8 @@ struct BatchRec {
     NetOut n;
     RadOut ro;
     View3<double> frazil;
-    uint8_t* freeze_flags;  // the member's freeze flags (written by stage 3, read by K2)
-    double* residual;       // the member's rounding residual (running totals per tile)
+    uint8_t* freeze_flags;  // the member's freeze flags (set by stage 3, read and cleared by K1)
+    double* residual;       // the member's rounding residual (running totals per tile and chunk of levels)
     const double* beer;     // the member's Beer's-law factors (two-colour forcing)
     int levels;             // levels per block of the stages (stage_levels)
     const double* atimes;   // device copies of the snapshot times

@@ -649,7 +649,7 @@ __global__ void radiation_kernel(GridDev g, ne_params p, View3<const double> sw,
     if (r.down_sw.p) r.down_sw.at2(i, j) = -Itsw;
 }
 
-// One column of K2: freeze clamp, net-flux assembly and radiation.
+// What finishes one column of K1: freeze clamp, net-flux assembly and radiation.
 template <typename Real, bool UNIT>
 __device__ __forceinline__ void surface_finalize_column(const GridDev& g, const ne_params& p, const View3<Real>& T,
                                                         const View3<const Real>& S, const NetOut& n, const RadOut& ro,
@@ -787,9 +787,9 @@ __global__ void __launch_bounds__(BX* BY) surface_tau_kernel(GridDev g, ne_param
 }
 
 // Ensemble form of K1: a persistent grid walks the (member, first column) work list; an
-// item is blockDim.x consecutive columns (i fastest) of one member. Members with the
-// default Edson constants are listed for the shared-ψ instance (Fast), the others for
-// the general one, as the single-model launcher chooses.
+// item is blockDim.x consecutive columns (i fastest) of one member. There is a list, and a launch, for
+// each flux path that members have (flux_path), as the single-model launcher chooses its instance; UNIT
+// holds for all members or for none.
 // FUSED (the step): each column then goes on as in the single model's K1 (freeze clamp of the
 // flagged columns, net fluxes other than τ, radiation); without it (the autotuner's timing
 // runs) the kernel only solves, leaving the state as it is.
@@ -838,7 +838,7 @@ batch_surface_solve_kernel(const BatchRec<Real>* __restrict__ recs, const WorkIt
     add_wave_counts(counters, n_it, n_solved, n_nc, n_nan, n_max);
 }
 
-// Ensemble form of K2 over the same work list as the ensemble K1: τ of every column.
+// Ensemble form of the τ kernel over the same work list as the ensemble K1: τ of every column.
 template <typename Real>
 __global__ void __launch_bounds__(BX* BY)
 batch_surface_tau_kernel(const BatchRec<Real>* __restrict__ recs, const WorkItem* __restrict__ work, int nwork) {
@@ -1113,7 +1113,7 @@ hipError_t launch_radiation(const GridDev& g, const ne_params& p, View3<const do
 }
 
 // The parameters for which the FP32 form's flux solve runs its FP32 iteration (flux_column,
-// Mixed && Fast): every column then either finishes in FP32 or is deferred.
+// Mixed, paths 1 to 3): every column then either finishes in FP32 or is deferred.
 bool mixed_iteration_applies(const ne_params& p) {
     const bool shared_scalar = p.temperature_roughness == p.water_vapor_roughness &&
                                (p.temperature_roughness == NE_ROUGHNESS_EDSON ||
